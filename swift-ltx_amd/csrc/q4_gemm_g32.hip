@@ -1,0 +1,11 @@
+// q4_gemm_g32.hip -- the fast GEMM kernels of group size 32.
+#include "q4_gemm_launch.hpp"
+
+namespace sltx {
+
+void launch_gemm_fast_g32(const GemmParams& p, bool bf16, bool silu, bool split, int wm, long grid,
+                          hipStream_t st) {
+    launch_gemm_fast<0>(p, bf16, silu, split, wm, grid, st);
+}
+
+}  // namespace sltx

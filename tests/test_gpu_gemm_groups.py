@@ -1,0 +1,67 @@
+"""The GEMM's fast kernel at group sizes 32 and 128 (scale / bias dwords copied
+direct to LDS) against its generic kernel, which stages them through registers
+and which a scale array at an odd 2-byte address selects: the same plan, k
+order and dequantization, so the results must be equal bit for bit.  The
+generic kernel is held to the oracle in test_gpu_gemm.py; one case here is too.
+
+K covers one and several super-stages (128 k), odd counts of them, and at
+group 128 splits that begin on the second group of a scale dword; M and N
+cover partial tiles, split, single-round and persistent launches."""
+import numpy as np
+import pytest
+
+from helpers import TOL_GEMM_F16, assert_parity, gpu_inputs, host
+from oracle import q4_oracle as o
+
+pytestmark = pytest.mark.gpu
+
+
+def _odd(t):
+    """The same values at an address 2 bytes past a multiple of 4."""
+    import torch
+    buf = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)
+    v = buf[1:1 + t.numel()].view(t.shape)
+    v.copy_(t)
+    assert v.data_ptr() % 4 == 2
+    return v
+
+
+# (300, 500, 1280) splits K; (1000, 16384, 512) runs persistent blocks
+SHAPES = [(257, 256, 256), (300, 500, 1280), (300, 777, 3328), (513, 3072, 3072), (700, 1000, 768),
+          (1000, 16384, 512)]
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_fast_equals_generic(pkg, dev, M, N, K, g):
+    import torch
+    for dt in ("f16", "bf16"):
+        x, [(w, s, b)] = gpu_inputs(M, N, K, g, seed=M + N + K, dev=dev, x_dtype=dt)
+        fast = pkg.matmul_q4_ex(x, pkg.Q4Weight(w, s, b, K, g), M, N)
+        gen = pkg.matmul_q4_ex(x, pkg.Q4Weight(w, _odd(s), _odd(b), K, g), M, N)
+        torch.cuda.synchronize()
+        assert torch.equal(fast, gen), f"{dt} M={M} N={N} K={K} g={g}"
+
+
+@pytest.mark.parametrize("g", [32, 128])
+@pytest.mark.parametrize("M,N,K", [(300, 200, 512), (700, 8192, 768), (500, 384, 3072)])
+def test_fast_equals_generic_pair(pkg, dev, M, N, K, g):
+    import torch
+    x, sets = gpu_inputs(M, N, K, g, seed=M + K, dev=dev, n_weights=2)
+    fast = pkg.matmul_q4_silu_mul(x, *(pkg.Q4Weight(*t, K, g) for t in sets), M, K, N)
+    gen = pkg.matmul_q4_silu_mul(x, *(pkg.Q4Weight(w, _odd(s), _odd(b), K, g) for w, s, b in sets),
+                                 M, K, N)
+    torch.cuda.synchronize()
+    assert torch.equal(fast, gen)
+
+
+@pytest.mark.parametrize("g", [32, 128])
+def test_fast_oracle(pkg, dev, g):
+    import torch
+    M, N, K = 400, 600, 1280
+    x, [(w, s, b)] = gpu_inputs(M, N, K, g, seed=g, dev=dev)
+    y = pkg.matmul_q4_fast_f32(x, w, s, b, M, K, N, g)
+    torch.cuda.synchronize()
+    rows = np.array([0, 127, 128, M - 1])
+    ref = o.matmul_q4_f64(host(x)[rows].astype(np.float64), host(w), host(s), host(b), g)
+    assert_parity(y.cpu().numpy()[rows], ref, TOL_GEMM_F16, f"g={g}")
