@@ -889,6 +889,32 @@ int sltx_matmul_q4_residual_rms_norm(const void* x, const sltx_q4_weight* w, con
         return fail(kErrInvalid,
                     "%s: no workspace on this stream (it is being captured: call it once eagerly "
                     "on the same stream first)", fn);
+    // Few rows: the weight streams and the wide route, then the row norm.  The
+    // GEMM pads M to 128 rows and writes up to six fp32 partial tiles for the
+    // fused pass.  Measured (us, both launches, weights rotated) against it:
+    // Llama o 7.4 / 8.7 / 10.2 / 15.6 / 19.7 / 22.1 against 17.2 / 17.9 / 18.6 /
+    // 19.6 / 23.6 / 27.0 at M = 2 / 8 / 32 / 64 / 128 / 256; Llama down 10.4 /
+    // 13.7 / 15.8 / 19.5 / 24.8 / 33.0 against 23.2 / 23.6 / 24.7 / 26.2 / 29.8 /
+    // 33.7.  (Under capture without a workspace the call has already failed,
+    // as it does for every shape.)
+    NarrowPlan np;
+    SkinnyPlan sp;
+    WidePlan wp;
+    if (gemm_route(p, false, &np, &sp, &wp) != SLTX_ROUTE_GEMM) {
+        // the projection in fp16 (norm_out holds it until the norm overwrites it in
+        // place) or, rounded, the summed stream
+        const uint16_t* proj = static_cast<const uint16_t*>(sum_rounded ? residual_out : norm_out);
+        rc = run_gemm(fn, x, kF16, *w, nullptr, nullptr, sum_rounded ? kEpiResidual : kEpiNone,
+                      sum_rounded ? residual_out : norm_out, kF16, M, w->K, N, st,
+                      sum_rounded ? residual : nullptr);
+        if (rc != kOk) return rc;
+        return finish(sum_rounded ? launch_rms_norm(proj, nullptr, norm_weight, eps, nullptr,
+                                                    static_cast<uint16_t*>(norm_out), M, N, st)
+                                  : launch_rms_norm(static_cast<const uint16_t*>(residual), proj, norm_weight,
+                                                    eps, static_cast<uint16_t*>(residual_out),
+                                                    static_cast<uint16_t*>(norm_out), M, N, st),
+                      fn);
+    }
     return finish(launch_gemm_residual_rms_norm(p, false, norm_weight, eps,
                                                 static_cast<uint16_t*>(residual_out),
                                                 static_cast<uint16_t*>(norm_out), sum_rounded != 0, st),
