@@ -2,8 +2,10 @@
 Ops entry points over the C ABI in include/swiftltx_q4.h.
 
 The shipped compute path is libswiftltx_q4.so (hand-written HIP for gfx950);
-this module only marshals torch device tensors into it with ctypes.  There is
-no fallback: if the library is missing, every entry point raises.
+this module only marshals torch device tensors into it: plain calls through
+lib/_q4_binding.so (csrc/py/q4_binding.cpp), everything else, and every error,
+through ctypes.  There is no fallback for the library: if it is missing, every
+entry point raises.
 
 Reference interface mirrored (Sources/SwiftLLM/ of swift-ltx):
     matmulQ4        Ops.swift:285-305      -> matmul_q4
@@ -189,6 +191,37 @@ def lib():
     return _lib
 
 
+# The native binding of the hot calls (csrc/py/q4_binding.cpp), loaded by the
+# first call on a torch tensor: each of its functions returns its Python
+# counterpart's result, or None for anything but the plain accepted call, which
+# then goes on in Python.  A matmul_q4 call took 12 us of host time through
+# ctypes (kernel: 3.3 us), a layer of five calls 73 us.
+BINDING_PATH = os.path.join(PKG_DIR, "lib", "_q4_binding.so")
+_native = None
+_native_tried = False
+
+
+def _load_binding():
+    global _native, _native_tried
+    _native_tried = True
+    if not os.path.exists(BINDING_PATH):
+        return
+    import importlib.util
+    import warnings
+    _torch()   # the binding links against its libraries (and the library takes its HIP runtime)
+    L = lib()
+    try:
+        spec = importlib.util.spec_from_file_location("_q4_binding", BINDING_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.init({n: ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in EXPORTED
+                  if not n.startswith("sltx_st_")}, check, Q4Weight)
+    except (ImportError, KeyError) as e:   # built against another torch: ctypes serves every call
+        warnings.warn(f"{BINDING_PATH} not loaded: {e}")
+        return
+    _native = mod
+
+
 def check(rc: int) -> None:
     if rc != SLTX_OK:
         msg = lib().sltx_last_error().decode(errors="replace")
@@ -218,6 +251,8 @@ def _ptr(t) -> int | None:
 
 def _stream(stream) -> int | None:
     torch = _torch()
+    if not _native_tried:
+        _load_binding()
     if stream is None:
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, int):
@@ -313,6 +348,10 @@ def _need_raw(weight, scales, biases, N, K, g):
 
 def matmul_q4(x, weight, scales, biases, M, K, N, group_size, out=None, stream=None):
     """matmulQ4 (Ops.swift:285-305): [M,N] fp16 = x[M,K] fp16 . dequant(W)^T."""
+    if _native is not None:
+        r = _native.matmul_q4(x, weight, scales, biases, M, K, N, group_size, out, stream)
+        if r is not None:
+            return r
     out = _new((M, N), _torch().float16, x) if out is None else out
     if M > 0 and N > 0 and _shape_ok(K, group_size):
         _need(x, "x", M * K, _f16())
@@ -325,6 +364,10 @@ def matmul_q4(x, weight, scales, biases, M, K, N, group_size, out=None, stream=N
 
 def matmul_q4_fast(x, weight, scales, biases, M, K, N, group_size, out=None, stream=None):
     """matmulQ4Fast (Ops.swift:312-345): MFMA GEMM, fp16 out."""
+    if _native is not None:
+        r = _native.matmul_q4_fast(x, weight, scales, biases, M, K, N, group_size, out, stream)
+        if r is not None:
+            return r
     out = _new((M, N), _torch().float16, x) if out is None else out
     if M > 0 and N > 0 and _shape_ok(K, group_size):
         _need(x, "x", M * K, _f16())
@@ -337,6 +380,10 @@ def matmul_q4_fast(x, weight, scales, biases, M, K, N, group_size, out=None, str
 
 def matmul_q4_fast_f32(x, weight, scales, biases, M, K, N, group_size, out=None, stream=None):
     """matmulQ4FastF32 (Ops.swift:348-381): MFMA GEMM, fp32 out."""
+    if _native is not None:
+        r = _native.matmul_q4_fast_f32(x, weight, scales, biases, M, K, N, group_size, out, stream)
+        if r is not None:
+            return r
     out = _new((M, N), _torch().float32, x) if out is None else out
     if M > 0 and N > 0 and _shape_ok(K, group_size):
         _need(x, "x", M * K, _f16())
@@ -349,6 +396,10 @@ def matmul_q4_fast_f32(x, weight, scales, biases, M, K, N, group_size, out=None,
 
 def silu_mul(a, b, out=None, stream=None):
     """siluMul (Ops.swift:44-56): half(silu(a) * b), fp16."""
+    if _native is not None:
+        r = _native.silu_mul(a, b, out, stream)
+        if r is not None:
+            return r
     out = _torch().empty_like(a) if out is None else out
     n = a.numel()
     if n > 0:
@@ -361,6 +412,10 @@ def silu_mul(a, b, out=None, stream=None):
 
 def linear(x, w: Q4Weight, M, K, N, fast=False, out=None, stream=None):
     """linear (Ops.swift:741-752), quantized case: fast && M>1 -> GEMM, else matmul_q4."""
+    if _native is not None:
+        r = _native.linear(x, w, M, K, N, fast, out, stream)
+        if r is not None:
+            return r
     out = _new((M, N), _torch().float16, x) if out is None else out
     if M > 0 and N > 0 and _shape_ok(K, w.group_size) and w.K == K:
         _need(x, "x", M * K, _f16())
@@ -375,6 +430,10 @@ def linear(x, w: Q4Weight, M, K, N, fast=False, out=None, stream=None):
 def matmul_q4_silu_mul(x, gate: Q4Weight, up: Q4Weight, M, K, N, out=None, stream=None):
     """Fused silu(x.Wg^T) * (x.Wu^T) -> fp16 [M, N]; replaces linear(gate),
     linear(up), siluMul (LlamaModel.swift:275-277, :327-329)."""
+    if _native is not None:
+        r = _native.matmul_q4_silu_mul(x, gate, up, M, K, N, out, stream)
+        if r is not None:
+            return r
     out = _new((M, N), _torch().float16, x) if out is None else out
     if M > 0 and N > 0 and _shape_ok(K, gate.group_size):
         _need(x, "x", M * K, _f16())
@@ -393,6 +452,10 @@ def matmul_q4_ex(x, w: Q4Weight, M, N, out_dtype=None, bias=None, epilogue=SLTX_
     fp16/bf16/fp32 (DiTLinear.applyF32in q4 branch, DiTModel.swift:102-125,
     + GELU-tanh); fp32 x is cast to fp16 with the +-65504 clamp of
     cast_f32_to_f16 (Kernels.swift:816-822) inside the GEMM."""
+    if _native is not None:
+        r = _native.matmul_q4_ex(x, w, M, N, out_dtype, bias, epilogue, out, stream)
+        if r is not None:
+            return r
     torch = _torch()
     if out is None:
         out = _new((M, N), out_dtype or torch.float32, x)
@@ -411,6 +474,10 @@ def matmul_q4_ex(x, w: Q4Weight, M, N, out_dtype=None, bias=None, epilogue=SLTX_
 
 def rms_norm(x, weight, eps, rows, dim, out=None, stream=None):
     """rmsNorm (Ops.swift:8-27): fp16 [rows, dim], fp32 weight [dim]."""
+    if _native is not None:
+        r = _native.rms_norm(x, weight, eps, rows, dim, out, stream)
+        if r is not None:
+            return r
     out = _new((rows, dim), _torch().float16, x) if out is None else out
     if rows > 0 and dim > 0:
         _need(x, "x", rows * dim, _f16())
@@ -423,6 +490,10 @@ def rms_norm(x, weight, eps, rows, dim, out=None, stream=None):
 def residual_rms_norm(a, b, weight, eps, rows, dim, residual_out=None, norm_out=None,
                       stream=None):
     """residualRmsNorm (Ops.swift:256-279) -> (residual, normed), fp16 [rows, dim]."""
+    if _native is not None:
+        r = _native.residual_rms_norm(a, b, weight, eps, rows, dim, residual_out, norm_out, stream)
+        if r is not None:
+            return r
     torch = _torch()
     residual_out = _new((rows, dim), torch.float16, a) if residual_out is None else residual_out
     norm_out = _new((rows, dim), torch.float16, a) if norm_out is None else norm_out
@@ -438,6 +509,10 @@ def residual_rms_norm(a, b, weight, eps, rows, dim, residual_out=None, norm_out=
 def rmsnorm_matmul_q4(x, norm_weight, eps, w: Q4Weight, N, out=None, stream=None):
     """rms_norm(x) . dequant(W)^T at M = 1 (input_layernorm + q|k|v,
     LlamaModel.swift:288-292) -> fp16 [1, N]."""
+    if _native is not None:
+        r = _native.rmsnorm_matmul_q4(x, norm_weight, eps, w, N, out, stream)
+        if r is not None:
+            return r
     out = _new((1, N), _torch().float16, x) if out is None else out
     if N > 0 and _shape_ok(w.K, w.group_size):
         _need(x, "x", w.K, _f16())
@@ -454,6 +529,11 @@ def residual_rmsnorm_matmul_q4_silu_mul(a, b, norm_weight, eps, gate: Q4Weight, 
                                         residual_out=None, out=None, stream=None):
     """residualRmsNorm + gate/up + siluMul at M = 1 (LlamaModel.swift:326-329)
     -> (residual [1, K], activated [1, N])."""
+    if _native is not None:
+        r = _native.residual_rmsnorm_matmul_q4_silu_mul(a, b, norm_weight, eps, gate, up, N, residual_out, out,
+                                                       stream)
+        if r is not None:
+            return r
     torch = _torch()
     residual_out = _new((1, gate.K), torch.float16, a) if residual_out is None else residual_out
     out = _new((1, N), torch.float16, a) if out is None else out
@@ -474,6 +554,10 @@ def residual_rmsnorm_matmul_q4_silu_mul(a, b, norm_weight, eps, gate: Q4Weight, 
 def matmul_q4_residual(x, w: Q4Weight, residual, M, N, out=None, stream=None):
     """half(residual + half(x . dequant(W)^T)): linear + elemAdd
     (LlamaModel.swift:330-331) -> fp16 [M, N]."""
+    if _native is not None:
+        r = _native.matmul_q4_residual(x, w, residual, M, N, out, stream)
+        if r is not None:
+            return r
     out = _new((M, N), _torch().float16, x) if out is None else out
     if M > 0 and N > 0 and _shape_ok(w.K, w.group_size):
         _need(x, "x", M * w.K, _f16())
@@ -494,6 +578,11 @@ def matmul_q4_residual_rms_norm(x, w: Q4Weight, residual, norm_weight, eps, M, N
     step's residualRmsNorm, LlamaModel.swift:269-272) or over residual_out
     (True: elemAdd then the next layer's rmsNorm, LlamaModel.swift:278-279, 233)
     -> (residual_out, norm_out), fp16 [M, N]."""
+    if _native is not None:
+        r = _native.matmul_q4_residual_rms_norm(x, w, residual, norm_weight, eps, M, N, sum_rounded,
+                                               residual_out, norm_out, stream)
+        if r is not None:
+            return r
     torch = _torch()
     residual_out = _new((M, N), torch.float16, x) if residual_out is None else residual_out
     norm_out = _new((M, N), torch.float16, x) if norm_out is None else norm_out
@@ -528,6 +617,10 @@ def gemm_route(M, N, K, group_size=64, gated=False, x_dtype=None):
 def matmul_q4_geglu(x, gate: Q4Weight, up: Q4Weight, M, K, N, out=None, stream=None):
     """gelu_tanh(x.Wg^T) * (x.Wu^T) -> fp16 [M, N]: the T5 encoder FFN's
     gate/up (T5Encoder.swift:191-199)."""
+    if _native is not None:
+        r = _native.matmul_q4_geglu(x, gate, up, M, K, N, out, stream)
+        if r is not None:
+            return r
     out = _new((M, N), _torch().float16, x) if out is None else out
     if M > 0 and N > 0 and _shape_ok(K, gate.group_size):
         _need(x, "x", M * K, _f16())
@@ -543,6 +636,10 @@ def matmul_q4_geglu(x, gate: Q4Weight, up: Q4Weight, M, K, N, out=None, stream=N
 def embedding_q4(table: Q4Weight, vocab, token_ids, out=None, stream=None):
     """embeddingQ4Batch (Ops.swift:163-187): dequantized rows [n, K] fp16 of a
     4-bit table for int32 device token ids."""
+    if _native is not None:
+        r = _native.embedding_q4(table, vocab, token_ids, out, stream)
+        if r is not None:
+            return r
     n = int(token_ids.numel())
     out = _new((n, table.K), _torch().float16, token_ids) if out is None else out
     if n > 0 and vocab >= 0 and _shape_ok(table.K, table.group_size):
@@ -567,6 +664,10 @@ def _logits_dtype(logits):
 def argmax(logits, out=None, stream=None):
     """argmax (Ops.swift:757-781) on the device: int32 [1] tensor holding the
     first index of the maximum of a contiguous fp16/fp32 vector."""
+    if _native is not None:
+        r = _native.argmax(logits, out, stream)
+        if r is not None:
+            return r
     out = _new((1,), _torch().int32, logits) if out is None else out
     _need(logits, "logits", logits.numel())
     _need(out, "out", 1, (_torch().int32,))
@@ -584,6 +685,11 @@ def sample(logits, temperature=0.7, top_p=0.9, repetition_penalty=1.1, seen_toke
     import random
     if u is None:
         u = random.random()
+    if _native is not None:
+        r = _native.sample(logits, temperature, top_p, repetition_penalty, seen_tokens, u, out,
+                           stream)
+        if r is not None:
+            return r
     out = _new((1,), _torch().int32, logits) if out is None else out
     n_seen = 0 if seen_tokens is None else int(seen_tokens.numel())
     _need(logits, "logits", logits.numel())

@@ -6,6 +6,9 @@
 csrc/*.hip -> lib/libswiftltx_q4.so, the drop-in library (include/swiftltx_q4.h).
 csrc/bench/*.hip -> lib/libswiftltx_bench.so, measurement kernels that only
 bench.py loads (the HBM read ceiling); not part of the C ABI.
+csrc/py/q4_binding.cpp -> lib/_q4_binding.so, the native marshalling of the
+Python mirror's hot calls (a CPython extension over torch's C++ tensors; host
+code, built with g++ where torch is installed).
 Objects go to swift-ltx_amd/_build/, the libraries to swift-ltx_amd/lib/.
 Every HIP file is compiled for gfx950 only, with packed-fp32 instruction
 selection disabled (hipcc's host pass warns that it does not know the
@@ -15,9 +18,11 @@ from __future__ import annotations
 
 import concurrent.futures as cf
 import glob
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(PKG)
@@ -26,6 +31,8 @@ OBJ_DIR = os.path.join(PKG, "_build")
 LIB_DIR = os.path.join(PKG, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libswiftltx_q4.so")
 BENCH_LIB_PATH = os.path.join(LIB_DIR, "libswiftltx_bench.so")
+BINDING_SRC = os.path.join(CSRC, "py", "q4_binding.cpp")
+BINDING_PATH = os.path.join(LIB_DIR, "_q4_binding.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 DEVICE_FLAGS = [
@@ -52,11 +59,35 @@ def headers() -> list[str]:
 
 
 def is_stale() -> bool:
-    if not os.path.exists(LIB_PATH) or not os.path.exists(BENCH_LIB_PATH):
+    outputs = [LIB_PATH, BENCH_LIB_PATH] + ([BINDING_PATH] if torch_dir() else [])
+    if not all(os.path.exists(f) for f in outputs):
         return True
-    t = min(os.path.getmtime(LIB_PATH), os.path.getmtime(BENCH_LIB_PATH))
+    t = min(os.path.getmtime(f) for f in outputs)
     return any(os.path.getmtime(f) > t
-               for f in sources() + bench_sources() + headers() + [__file__])
+               for f in sources() + bench_sources() + headers() + [BINDING_SRC, __file__])
+
+
+def torch_dir() -> str | None:
+    """The installed torch's folder, found without importing it."""
+    spec = importlib.util.find_spec("torch")
+    return os.path.dirname(spec.origin) if spec and spec.origin else None
+
+
+def _build_binding() -> None:
+    t = torch_dir()
+    if not t:
+        return
+    tmp = BINDING_PATH + ".tmp%d" % os.getpid()
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           "-I" + os.path.join(REPO, "include"), "-I" + os.path.join(t, "include"),
+           "-I" + os.path.join(t, "include", "torch", "csrc", "api", "include"),
+           "-I" + sysconfig.get_paths()["include"], "-isystem", "/opt/rocm/include",
+           BINDING_SRC, "-o", tmp, "-L" + os.path.join(t, "lib"),
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for {BINDING_SRC}:\n{r.stderr}")
+    os.replace(tmp, BINDING_PATH)
 
 
 def _compile(src: str) -> str:
@@ -84,14 +115,16 @@ def _link(objs: list[str], path: str) -> None:
 
 def build(force: bool = True, jobs: int = 8) -> str:
     """Compile every csrc/*.hip (and csrc/bench/*.hip) for gfx950, link
-    LIB_PATH and BENCH_LIB_PATH; returns LIB_PATH."""
+    LIB_PATH and BENCH_LIB_PATH, and build BINDING_PATH; returns LIB_PATH."""
     if not force and not is_stale():
         return LIB_PATH
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     main, bench = sources(), bench_sources()
     with cf.ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
+        binding = ex.submit(_build_binding)
         objs = list(ex.map(_compile, main + bench))
+        binding.result()
     _link(objs[:len(main)], LIB_PATH)
     _link(objs[len(main):], BENCH_LIB_PATH)
     return LIB_PATH
