@@ -15,8 +15,8 @@
  *     frees or keeps them.  Outputs are written, never read.
  *   - Memory: the only device memory the library allocates is a per-stream
  *     workspace: fp32 partial sums for GEMMs with too few output tiles to
- *     fill the GPU (split-K, e.g. M=750 x N=3072, and at 8 < M <= 256 the
- *     mid- and wide-M K splits, e.g. M=32 x 4096 x 10240) and for every
+ *     fill the GPU (split-K, e.g. M=750 x N=3072, and the mid- and wide-M
+ *     K splits, e.g. M=32 x 4096 x 10240) and for every
  *     sltx_matmul_q4_residual_rms_norm, the block partials of
  *     sltx_argmax, and the probabilities and candidate list of
  *     sltx_sample_top_p[_state], after 16 KB of split-K arrival counters
@@ -349,8 +349,9 @@ typedef enum {
     SLTX_ROUTE_MID = 3,      /* pipelined weight stream (8 < M <= 32, from M = 6 for a set of at most
                                 4096 rows at K = 10240; X and W through LDS, 32x32x16 MFMA; such
                                 sets split K in halves across blocks) */
-    SLTX_ROUTE_WIDE = 4,     /* 32 < M <= 256: 64 weight rows per block over its K range, waves
-                                split K; K split across blocks where the blocks are few */
+    SLTX_ROUTE_WIDE = 4,     /* M > 32 where one round of blocks covers it: 64 weight rows per
+                                block over its K range, waves split K; K split across blocks
+                                where the blocks are few */
     SLTX_ROUTE_GEMV = 5      /* M = 2, fp16 x, one weight set of at most 5120 x 4096: the GEMV
                                 over both rows (each weight word dequantized once) */
 } sltx_route;

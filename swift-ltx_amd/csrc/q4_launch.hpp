@@ -197,7 +197,7 @@ int mid_splits(const GemmParams& p);
 size_t mid_ws_bytes(const GemmParams& p, int splits);
 hipError_t launch_mid(const GemmParams& p, int splits, hipStream_t st);
 
-// Wide-M route (q4_wide.hip, 32 < M <= 256, fp16 X): 64 weight rows (or a
+// Wide-M route (q4_wide.hip, M > 32, fp16 X, one round of blocks): 64 weight rows (or a
 // 32-row gate/up pair) per block over all of its K range, up to 128
 // activation rows per block (more rows take more blocks), the 8 waves
 // splitting K; optionally split over K across blocks (fp32 partials in the

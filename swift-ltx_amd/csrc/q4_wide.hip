@@ -1,6 +1,7 @@
-// q4_wide.hip -- 4-bit dequant matmul for 32 < M <= 256 activation rows
-// (T5 encoder layers at S <= 256, T5Encoder.swift:72-78 and :140-205; short
-// prompts) on CDNA4 MFMA.
+// q4_wide.hip -- 4-bit dequant matmul for M > 32 activation rows where its
+// grid is one round of blocks (T5 encoder layers at S <= 256,
+// T5Encoder.swift:72-78 and :140-205; prompts of up to some hundred tokens;
+// narrow projections of more) on CDNA4 MFMA.
 //
 // Same product as q4_gemm.hip, Y[M,N] = X[M,K] . dequant(W)[N,K]^T with fp32
 // accumulation (matmulQ4Fast, Ops.swift:312-381).  Between the mid-M weight
@@ -26,7 +27,7 @@
 //    compiler then knows that reads of one stage do not alias copies in
 //    flight into another.
 //  * The block's scales and biases (64 rows x its K range's groups, at most
-//    64 groups) are read once into an LDS slab as scale | bias << 16 words.
+//    128 groups) are read once into an LDS slab as scale | bias << 16 words.
 //  * After the last round the 8 waves' tiles are summed in LDS in a fixed
 //    order (one 32-row tile at a time) and the epilogue (gated SiLU /
 //    GELU-tanh, bias, GELU-tanh, residual add) runs on the fp32 sums.  With a
@@ -58,7 +59,7 @@ constexpr int WRD = RK / 8;         // packed words of a weight row per round (1
 constexpr int WDW = WBN * WRD;      // dwords of a W stage (1024)
 constexpr int WPC = WDW / 4;        // 16-byte W pieces per round (256)
 constexpr int WCW = WPC / 64;       // waves that copy them, one piece per lane (4)
-constexpr int SLAB_G = 64;          // scale / bias groups a block holds
+constexpr int SLAB_G = 128;         // scale / bias groups a block holds
 // Ring stages by tile height (a stage is BM x 256 bytes of X + 4 KB of W).
 // Measured over the Llama and T5 shapes at M = 33..256: at TM = 4 three
 // stages run 0.1-0.5 us faster than four; at TM = 2 six or seven stages
@@ -194,11 +195,12 @@ __global__ __launch_bounds__(WT, 1) void q4_wide_kernel(GemmParams p, WideArgs w
     static_assert(XS * 16 >= 2 * 8 * 1024, "two waves' 32-row tiles fit one X stage");
     // One array per stage (stage indices are compile-time, so the compiler
     // sees that reads of one stage do not alias copies into another).  The
-    // fourth X array exists at NSX = 3 too: the K-groups' sums are staged in
-    // all four.
-    __shared__ u32x4 xs0[XS], xs1[XS], xs2[XS], xs3[XS];
+    // K-groups' sums are staged in the four X arrays, at NSX = 3 in three of
+    // them and the slab.
+    __shared__ u32x4 xs0[XS], xs1[XS], xs2[XS], xs3[NSX > 3 ? XS : 1];
     __shared__ uint32_t ws0[WDW], ws1[WDW], ws2[WDW], ws3[NSX > 3 ? WDW : 1];
-    __shared__ uint32_t slab[SLAB_G * WBN];
+    __shared__ __align__(16) uint32_t slab[SLAB_G * WBN];
+    
     auto xstage = [&](auto sc) -> u32x4* {
         constexpr int S = decltype(sc)::value % NSX;
         if constexpr (S == 0) return xs0;
@@ -293,23 +295,45 @@ __global__ __launch_bounds__(WT, 1) void q4_wide_kernel(GemmParams p, WideArgs w
     const int glog2 = 5 + p.gshift;
     const int gbase = kb >> glog2;
     const int ng = wa.kblk >> glog2;    // groups of this block (<= SLAB_G)
-    constexpr int NSE = (WBN * SLAB_G + WT - 1) / WT;   // slab entries per thread (at most)
-    uint32_t sv[NSE], bv[NSE];
-#pragma unroll
-    for (int u = 0; u < NSE; ++u) {
-        const int e = tid + WT * u;
-        const int row = e / ng, gi = e % ng;
+    // Wave w fills rows 8 w .. 8 w + 7, lanes along a row's groups (contiguous
+    // reads, no division); up to 16 groups, four rows a load.
+    auto slab_row = [&](int row, const uint16_t*& S, const uint16_t*& B) {
         const uint32_t* W;
-        const uint16_t *S, *B;
-        const int n = wrow(e < WBN * ng ? row : 0, W, S, B);
-        const size_t o = (size_t)n * p.groups + gbase + (e < WBN * ng ? gi : 0);
-        sv[u] = S[o];
-        bv[u] = B[o];
-    }
+        const int n = wrow(row, W, S, B);
+        S += (size_t)n * p.groups + gbase;
+        B += (size_t)n * p.groups + gbase;
+    };
+    if (ng <= 16) {
+        const int gi = min(lane & 15, ng - 1);
+        uint32_t sv[2], bv[2];
 #pragma unroll
-    for (int u = 0; u < NSE; ++u) {
-        const int e = tid + WT * u;
-        if (e < WBN * ng) slab[spos(e % ng, e / ng)] = sv[u] | (bv[u] << 16);
+        for (int u = 0; u < 2; ++u) {
+            const uint16_t *S, *B;
+            slab_row(8 * wave + 4 * u + (lane >> 4), S, B);
+            sv[u] = S[gi];
+            bv[u] = B[gi];
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            if ((lane & 15) < ng) slab[spos(gi, 8 * wave + 4 * u + (lane >> 4))] = sv[u] | (bv[u] << 16);
+    } else {
+        uint32_t sv[16], bv[16];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const uint16_t *S, *B;
+            slab_row(8 * wave + u, S, B);
+            sv[u] = S[min(lane, ng - 1)];
+            bv[u] = B[min(lane, ng - 1)];
+            if (ng > 64) {
+                sv[8 + u] = S[min(64 + lane, ng - 1)];
+                bv[8 + u] = B[min(64 + lane, ng - 1)];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if (lane < ng) slab[spos(lane, 8 * wave + u)] = sv[u] | (bv[u] << 16);
+            if (64 + lane < ng) slab[spos(64 + lane, 8 * wave + u)] = sv[8 + u] | (bv[8 + u] << 16);
+        }
     }
 
     const int r = lane & 31, h = lane >> 5;
@@ -424,7 +448,8 @@ __global__ __launch_bounds__(WT, 1) void q4_wide_kernel(GemmParams p, WideArgs w
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
     WIDE_LDS_BARRIER();
     auto buf = [&](int w, int d) -> float* {
-        u32x4* st = (w >> 1) == 0 ? xs0 : (w >> 1) == 1 ? xs1 : (w >> 1) == 2 ? xs2 : xs3;
+        u32x4* st = (w >> 1) == 0 ? xs0 : (w >> 1) == 1 ? xs1 : (w >> 1) == 2 ? xs2
+                    : NSX > 3 ? xs3 : reinterpret_cast<u32x4*>(slab);
         return reinterpret_cast<float*>(st) + d * 4096 + (w & 1) * 2048;
     };
     constexpr int NV = PAIR ? 2 : 4;     // columns a thread sums
@@ -520,11 +545,34 @@ hipError_t launch_tm(const GemmParams& p, const WideArgs& wa, const dim3& grid, 
 
 }  // namespace
 
-// Plan: M-blocks of at most 128 rows (balanced), TM = the 32-row tiles of
-// one; K split across blocks when the blocks would not fill the GPU (and
-// until a block's K range holds at most 64 scale groups), in whole rounds.
+// Plan: M-blocks of 32 TM rows (TM = 2..4, balanced) and K splits (1, 2, 3, 4
+// or 8: the fix-up's instantiations), by estimated time.  A grid is at most
+// one round of 256 blocks: a second round repeats the whole per-block time
+// (gate/up + SiLU at M = 200: 45.7 us against the GEMM's 41.3, the T5 GeGLU
+// pair's 320 blocks at M = 128: 55.3 against 42.4), which still wins at M <=
+// 64 (that pair at M = 64: 34.8 against 37.3).
+//
+// The estimate, in us, from launches at K = 128..10240, M = 33..6144 and
+// 10..256 blocks (it is within 1 us of them): a fixed part (launch, first
+// memory latency, scale slab, cross-wave sum), a round of 128 k, dearer with
+// more rows and with more CUs pulling X from L2, and the splits' hand-off.
+// Against the tallest M-blocks that fit, as the plan was: o (3072 x 3072) at
+// M = 128 / 256 13.1 / 15.5 us (2 x 64 rows x 2 splits, 4 x 64 x 1) against
+// 15.6 / 17.4; 4096 x 4096 15.0 / 19.4 against 17.0 / 20.4; Llama down keeps
+// its 128-row blocks.
+//
+// Above 256 rows the GEMM's few 128- or 192-row tiles need K splits, whose
+// partials pass through HBM, so one round here is faster where a block's K is
+// at most 4096 and X (re-read by every 64 weight rows) stays in the Infinity
+// Cache.  Measured against the GEMM: o at M = 333 / 640 17.8 / 22.5 against
+// 27.0 / 30.7, q|k|v at M = 333 21.9 against 29.9, 2048 x 2048 at M = 1000
+// 17.7 against 29.0, 1024 x 4096 at M = 1000 20.0 against 28.9, 128 x 2048 at
+// M = 6144 (X 25 MB) 15.7 against 21.5.  Past those limits: 256 x 4096 at M =
+// 6144 (X 50 MB) 35.6 against 29.7; K = 8192 unsplit, 3072 rows at M = 500
+// 44.0 against 42.2, 2048 rows at M = 600 43.0 against 38.6.
 bool wide_plan(const GemmParams& p, bool a_bf16, WidePlan* out) {
-    if (a_bf16 || p.M <= 32 || p.M > 256 || p.N < 1) return false;
+    if (a_bf16 || p.M <= 32 || p.N < 1) return false;
+    if (p.M > 256 && (size_t)p.M * p.K * 2 > (size_t)32 << 20) return false;
     if (p.K <= 0 || p.K % RK != 0 || p.gshift < 0 || p.gshift > 2) return false;
     const bool pair = p.w1 != nullptr;
     if (pair && p.epilogue != kEpiSiluMul && p.epilogue != kEpiGeluMul) return false;
@@ -534,49 +582,40 @@ bool wide_plan(const GemmParams& p, bool a_bf16, WidePlan* out) {
     // 16-byte X pieces: 16-byte aligned X (K % 8 == 0 keeps every row so);
     // packed W moves as dwords
     if ((reinterpret_cast<uintptr_t>(p.a) & 15) != 0) return false;
-    WidePlan pl;
-    pl.mblocks = (p.M + 127) / 128;
-    pl.mrows = (p.M + pl.mblocks - 1) / pl.mblocks;
-    pl.tm = (pl.mrows + 31) / 32;
-    if (pl.tm < 2) pl.tm = 2;
-    pl.nblocks = (p.N + (pair ? 31 : WBN - 1)) / (pair ? 32 : WBN);
-    // Two M-blocks of up to 128 rows that fill 160-255 CUs where three
-    // fit one round: three, of up to 86 rows (Llama q|k|v, 80 blocks per
-    // M-block: 14.7 / 17.2 / 17.4 against 17.0 / 19.9 / 20.3 us at M = 160 /
-    // 200 / 256).
-    if (pl.mblocks == 2 && pl.nblocks * 2 >= 160 && pl.nblocks * 3 <= kCUs) {
-        pl.mblocks = 3;
-        pl.mrows = (p.M + 2) / 3;
-        pl.tm = (pl.mrows + 31) / 32;
-    }
     const int g = 32 << p.gshift;
     const int rounds = p.K / RK;
-    const long blocks = (long)pl.nblocks * pl.mblocks;
-    int s = 1;   // 1, 2, 3, 4 or 8 (the fix-up's instantiations)
-    while (s < 8 && rounds % (2 * s) == 0 &&
-           ((long)p.K / s / g > SLAB_G || (blocks * s < 160 && rounds / (2 * s) >= 4)))
-        s *= 2;
-    // Two splits that leave a quarter of the CUs idle, where three fit one
-    // round: three (Llama q|k|v, 80 blocks: 240 instead of 160; 11.2 / 11.8
-    // / 15.9 against 12.2 / 12.6 / 17.0 us at M = 33 / 64 / 128).
-    if (s < 3 && blocks * s < 192 && blocks * 3 <= kCUs && rounds % 3 == 0 && rounds / 3 >= 4 &&
-        (long)p.K / 3 / g <= SLAB_G)
-        s = 3;
-    if ((long)p.K / s / g > SLAB_G) return false;
-    // One block per CU: a grid of more than one round of 256 blocks repeats
-    // the whole per-block time.  Measured against the GEMM (us, weights
-    // rotated over >= 1.5 GB): one round wins on every Llama and T5 shape
-    // (e.g. gate/up + SiLU at M = 128: 24.9 against 33.5, T5 wo 26.2 against
-    // 30.8); two rounds lose at M >= 100 (gate/up at M = 200: 45.7 against
-    // 41.3, the T5 GeGLU pair's 320 blocks at M = 128: 55.3 against 42.4)
-    // and still win at M <= 64 (that pair at M = 64: 34.8 against 37.3).
-    const long grid = blocks * s;
-    if (grid > kCUs && !(p.M <= 64 && grid <= 2 * kCUs)) return false;
-    pl.splits = s;
-    pl.kblk = p.K / s;
-    pl.ws_bytes = s > 1 ? (size_t)s * p.M * (pair ? 2 : 1) * p.N * sizeof(float) : 0;
-    *out = pl;
-    return true;
+    // K of one block: a slab of at most SLAB_G groups, and no more than
+    // measured (4096; group 128 at M <= 256: 8192)
+    const int kmax = p.M <= 256 && g == 128 ? 8192 : 4096;
+    
+    const long nblocks = ((long)p.N + (pair ? 31 : WBN - 1)) / (pair ? 32 : WBN);
+    const long most = p.M <= 64 ? 2 * kCUs : kCUs;
+    double best_us = 1e30;
+    for (int tm = 2; tm <= 4; ++tm) {
+        const long mblocks = ((long)p.M + 32 * tm - 1) / (32 * tm);
+        const int mrows = (int)((p.M + mblocks - 1) / mblocks);
+        if ((mrows + 31) / 32 < tm && tm > 2) continue;   // the shorter tile has this plan
+        for (int s : {1, 2, 3, 4, 8}) {
+            const long grid = nblocks * mblocks * s;
+            if (grid > most || rounds % s != 0 || p.K / s > kmax || (s > 1 && rounds / s < 4)) continue;
+            if (s > 1 && nblocks * mblocks > kTickets) continue;
+            const double busy = (double)(grid < kCUs ? grid : kCUs) / kCUs;
+            const double fixed = 3.5 + tm, round = tm == 2 ? 0.40 + 0.05 * busy
+                                                : tm == 3 ? 0.43 + 0.09 * busy : 0.48 + 0.16 * busy;
+            const double us = (fixed + round * (rounds / s)) * (grid > kCUs ? 2 : 1) +
+                              (s == 1 ? 0.0 : s == 2 ? 2.6 : s == 3 ? 3.5 : s == 4 ? 4.4 : 7.0);
+            if (us >= best_us) continue;
+            best_us = us;
+            out->tm = tm;
+            out->mblocks = (int)mblocks;
+            out->mrows = mrows;
+            out->nblocks = (int)nblocks;
+            out->splits = s;
+            out->kblk = p.K / s;
+            out->ws_bytes = s > 1 ? (size_t)s * p.M * (pair ? 2 : 1) * p.N * sizeof(float) : 0;
+        }
+    }
+    return best_us < 1e30;
 }
 
 hipError_t launch_wide(GemmParams p, const WidePlan& pl, hipStream_t st) {
