@@ -252,9 +252,9 @@ int sltx_matmul_q4_residual(const void* x, const sltx_q4_weight* w, const void* 
  * norm_out = rms_norm(residual_out) with norm_weight (fp32 [N]); both equal,
  * bit for bit, the unfused sequence of this library's M > 1 product
  * (sltx_matmul_q4_fast, sltx_matmul_q4_residual) and sltx_residual_rms_norm /
- * sltx_rms_norm.  Where sltx_gemm_route names a route other than the GEMM
- * (any M >= 1) that route runs, then one row norm; where it names the GEMM,
- * its fp32 partial sums go through the per-stream workspace, then one pass
+ * sltx_rms_norm.  Any M >= 1: the product's own kernel (sltx_gemm_route), then
+ * one row norm; where that is the GEMM with K splits, its fp32 partial sums go
+ * through the per-stream workspace, then one pass adds them, adds and normalizes
  * per row.  N % 8 == 0 and N <= 16384; residual, residual_out, norm_out,
  * norm_weight 16-byte aligned.  residual_out may be residual (in place);
  * norm_out must overlap neither, and no output may overlap x.  While the stream

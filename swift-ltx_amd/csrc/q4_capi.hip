@@ -889,8 +889,9 @@ int sltx_matmul_q4_residual_rms_norm(const void* x, const sltx_q4_weight* w, con
         return fail(kErrInvalid,
                     "%s: no workspace on this stream (it is being captured: call it once eagerly "
                     "on the same stream first)", fn);
-    // Few rows: the weight streams and the wide route, then the row norm.  The
-    // GEMM pads M to 128 rows and writes up to six fp32 partial tiles for the
+    // Where the product needs no reduce pass (the weight streams, the wide
+    // route, an unsplit GEMM), it runs as it would alone, then the row norm.  The
+    // GEMM pads few rows to 128 and writes up to six fp32 partial tiles for the
     // fused pass.  Measured (us, both launches, weights rotated) against it:
     // Llama o 7.4 / 8.7 / 10.2 / 15.6 / 19.7 / 22.1 against 17.2 / 17.9 / 18.6 /
     // 19.6 / 23.6 / 27.0 at M = 2 / 8 / 32 / 64 / 128 / 256; Llama down 10.4 /
@@ -900,7 +901,7 @@ int sltx_matmul_q4_residual_rms_norm(const void* x, const sltx_q4_weight* w, con
     NarrowPlan np;
     SkinnyPlan sp;
     WidePlan wp;
-    if (gemm_route(p, false, &np, &sp, &wp) != SLTX_ROUTE_GEMM) {
+    if (gemm_route(p, false, &np, &sp, &wp) != SLTX_ROUTE_GEMM || gemm_splits(p) == 1) {
         // the projection in fp16 (norm_out holds it until the norm overwrites it in
         // place) or, rounded, the summed stream
         const uint16_t* proj = static_cast<const uint16_t*>(sum_rounded ? residual_out : norm_out);

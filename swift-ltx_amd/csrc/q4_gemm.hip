@@ -181,6 +181,17 @@ __global__ __launch_bounds__(256) void q4_splitk_residual_rms_norm_kernel(
     }
 }
 
+// The fixed-count kernel needs whole 128-k super-stages, and for group size
+// 128 whole pairs of them (scales and biases move as dword pairs of groups, so
+// their arrays must also be 4-byte aligned; 2-byte aligned ones take the
+// generic kernel, which reads them as 16-bit values), and 32-bit offsets
+// within a tile's rows.
+static bool fast_gemm(const GemmParams& p) {
+    const uintptr_t sb_addr = reinterpret_cast<uintptr_t>(p.s0) | reinterpret_cast<uintptr_t>(p.b0) |
+                              reinterpret_cast<uintptr_t>(p.s1) | reinterpret_cast<uintptr_t>(p.b1);
+    return !p.a_f32 && p.K <= (1 << 22) && p.K % (p.gshift == 2 ? 4 * BK : 2 * BK) == 0 && (sb_addr & 3) == 0;
+}
+
 // Launch plan: block-tile height WM (BM = 64*WM) and K splits, chosen by
 // estimated time on 256 CUs: rounds of blocks x (k-tiles per block x the
 // measured time of one k-tile -- 1.37 us at BM = 192, 0.95 us at BM = 128,
@@ -188,31 +199,37 @@ __global__ __launch_bounds__(256) void q4_splitk_residual_rms_norm_kernel(
 // repeats) + ~2 us per launch, plus, when split, writing the fp32 partials
 // (~6 TB/s) and the reduce pass reading them back (~4 TB/s, its own launch).
 // Measured at M = 750 (lm_head, N = 128256): 664 us at BM = 192 vs 730 us at
-// BM = 128; DiT up (M = 6144, bf16): 318 vs 356 us.  Splits cover an even
+// BM = 128; DiT up (M = 6144, bf16): 318 vs 356 us.  Tiles of 128 x 128
+// (kg = 2, the fast kernel) are for single rounds where 256-row weight tiles
+// would leave CUs idle or split K.  Measured, kg = 2 against the best kg = 1
+// plan: q|k|v at M = 750 (240 blocks against 120 in two splits) 33.5 / 42.4 us,
+// gate/up at M = 200 32.0 / 40.9, 2048 x 2048 at M = 1537 23.0 / 30.9, 4096 x
+// 4096 at M = 1000 47.5 / 52.7; long K turns it round: down at M = 750 64 / 55,
+// 2048 x 8192 at M = 1537 76 / 71, the T5 GeGLU pair at M = 128 45.5 / 42.2.
+// Its 0.62 us per k-tile (0.55 measured) puts the line between those.  Splits cover an even
 // number of k-tiles (packed weights move two k-tiles at a time).
 struct GemmPlan {
-    int wm, tiles_m, tiles_n, splits, split_tiles;
+    int wm, kg, tiles_m, tiles_n, splits, split_tiles;
     size_t ws_bytes;
 };
 
-// partials: the output goes through the fp32 workspace at every split count
-// (including one), because a row-wise pass follows (the fused residual +
-// RMSNorm), so the unsplit plan pays the partial traffic too.
-static GemmPlan plan_gemm(const GemmParams& p, bool allow_split, bool partials = false) {
+static GemmPlan plan_gemm(const GemmParams& p, bool allow_split) {
     const bool silu = p.epilogue == kEpiSiluMul || p.epilogue == kEpiGeluMul;
-    const int bn_out = silu ? BN / 2 : BN;
-    const int tiles_n = (p.N + bn_out - 1) / bn_out;
     const int nk = (p.K + BK - 1) / BK;
     const size_t nw = silu ? 2 * (size_t)p.N : (size_t)p.N;
-    GemmPlan best = {2, 0, tiles_n, 1, nk, 0};
+    GemmPlan best = {2, 1, 0, 0, 1, nk, 0};
     double best_us = 1e30;
-    // fp32 activations hold a k-tile of A in registers: the 192-row tile
-    // would spill, so they take the 128-row tile only
-    for (int wm = 2; wm <= (p.a_f32 ? 2 : 3); ++wm) {
-        const int bm = 64 * wm;
+    const bool fast = fast_gemm(p);
+    static const struct { int wm, kg; double kt_us; } kTiles[] = {{2, 1, 0.95}, {3, 1, 1.37}, {2, 2, 0.62}};
+    for (const auto& t : kTiles) {
+        // fp32 activations hold a k-tile of A in registers: the 192-row tile
+        // would spill, so they take the 128-row tile only
+        if ((p.a_f32 && t.wm > 2) || (t.kg > 1 && !fast)) continue;
+        const int wm = t.wm, bm = 64 * wm, bn_out = BN / t.kg / (silu ? 2 : 1);
+        const long tiles_n = ((long)p.N + bn_out - 1) / bn_out;
         const long tiles_m = (p.M + bm - 1) / bm;
         const long tiles = tiles_m * tiles_n;
-        const double kt_us = wm == 3 ? 1.37 : 0.95;
+        const double kt_us = t.kt_us;
         const int smax = allow_split ? 8 : 1;
         for (int s = 1; s <= smax; ++s) {
             if (s > 1 && nk < 8 * s) break;
@@ -221,16 +238,17 @@ static GemmPlan plan_gemm(const GemmParams& p, bool allow_split, bool partials =
             const int s_eff = (nk + chunk - 1) / chunk;
             if (s > 1 && s_eff != s) continue;
             const long blocks = tiles * s_eff;
+            if (t.kg > 1 && blocks > kCUs) break;
             const long rounds = (blocks + kCUs - 1) / kCUs;
             double us = (double)rounds * (chunk * kt_us + 8.0) + 2.0;
-            const bool ws = s_eff > 1 || partials;
+            const bool ws = s_eff > 1;
             if (ws) {
                 const double part = (double)s_eff * p.M * nw * 4.0;
                 us += part / 6.0e6 + 3.0 + (part + (double)p.M * p.N * 2.0) / 4.0e6;
             }
             if (us < best_us) {
                 best_us = us;
-                best = {wm, (int)tiles_m, tiles_n, s_eff, chunk,
+                best = {wm, t.kg, (int)tiles_m, (int)tiles_n, s_eff, chunk,
                         ws ? (size_t)s_eff * p.M * nw * sizeof(float) : 0};
             }
         }
@@ -239,12 +257,15 @@ static GemmPlan plan_gemm(const GemmParams& p, bool allow_split, bool partials =
 }
 
 size_t gemm_workspace_bytes(const GemmParams& p) { return plan_gemm(p, true).ws_bytes; }
-size_t gemm_partials_workspace_bytes(const GemmParams& p) { return plan_gemm(p, true, true).ws_bytes; }
+int gemm_splits(const GemmParams& p) { return plan_gemm(p, true).splits; }
+size_t gemm_partials_workspace_bytes(const GemmParams& p) {
+    return (size_t)gemm_splits(p) * p.M * p.N * sizeof(float);
+}
 
 // The fast kernel's launcher of each group size, one translation unit each
 // (q4_gemm_g32.hip, q4_gemm_g64.hip, q4_gemm_g128.hip).
 template <int WM, bool BF16, bool SPLIT>
-static void launch_wm(const GemmParams& p, bool silu, long grid, hipStream_t st) {
+static void launch_wm(const GemmParams& p, bool silu, int kg, long grid, hipStream_t st) {
     if constexpr (WM == 2) {
         if (p.a_f32) {
             hipLaunchKernelGGL((q4_gemm_kernel<2, false, false, true, SPLIT, true>), dim3(grid),
@@ -252,16 +273,10 @@ static void launch_wm(const GemmParams& p, bool silu, long grid, hipStream_t st)
             return;
         }
     }
-    // The fixed-count kernel needs whole 128-k super-stages, and for group
-    // size 128 whole pairs of them (scales and biases move as dword pairs of
-    // groups, so their arrays must also be 4-byte aligned; 2-byte aligned
-    // ones take the generic kernel, which reads them as 16-bit values).
-    const uintptr_t sb_addr = reinterpret_cast<uintptr_t>(p.s0) | reinterpret_cast<uintptr_t>(p.b0) |
-                              reinterpret_cast<uintptr_t>(p.s1) | reinterpret_cast<uintptr_t>(p.b1);
-    if (p.K % (p.gshift == 2 ? 4 * BK : 2 * BK) == 0 && (sb_addr & 3) == 0) {
-        if (p.gshift == 0) launch_gemm_fast_g32(p, BF16, silu, SPLIT, WM, grid, st);
-        else if (p.gshift == 1) launch_gemm_fast_g64(p, BF16, silu, SPLIT, WM, grid, st);
-        else launch_gemm_fast_g128(p, BF16, silu, SPLIT, WM, grid, st);
+    if (fast_gemm(p)) {
+        if (p.gshift == 0) launch_gemm_fast_g32(p, BF16, silu, SPLIT, WM, kg, grid, st);
+        else if (p.gshift == 1) launch_gemm_fast_g64(p, BF16, silu, SPLIT, WM, kg, grid, st);
+        else launch_gemm_fast_g128(p, BF16, silu, SPLIT, WM, kg, grid, st);
         return;
     }
     if (silu)
@@ -271,14 +286,14 @@ static void launch_wm(const GemmParams& p, bool silu, long grid, hipStream_t st)
 }
 
 template <bool SPLIT>
-static void launch_dtype(const GemmParams& p, bool a_bf16, bool silu, long grid, int wm,
+static void launch_dtype(const GemmParams& p, bool a_bf16, bool silu, long grid, const GemmPlan& pl,
                          hipStream_t st) {
     if (a_bf16) {
-        if (wm == 2) launch_wm<2, true, SPLIT>(p, silu, grid, st);
-        else launch_wm<3, true, SPLIT>(p, silu, grid, st);
+        if (pl.wm == 2) launch_wm<2, true, SPLIT>(p, silu, pl.kg, grid, st);
+        else launch_wm<3, true, SPLIT>(p, silu, pl.kg, grid, st);
     } else {
-        if (wm == 2) launch_wm<2, false, SPLIT>(p, silu, grid, st);
-        else launch_wm<3, false, SPLIT>(p, silu, grid, st);
+        if (pl.wm == 2) launch_wm<2, false, SPLIT>(p, silu, pl.kg, grid, st);
+        else launch_wm<3, false, SPLIT>(p, silu, pl.kg, grid, st);
     }
 }
 
@@ -323,10 +338,10 @@ hipError_t launch_gemm(GemmParams p, bool a_bf16, hipStream_t st) {
     const long grid = (blocks + 7) / 8 * 8;
     if (grid > 0x7fffffffL) return hipErrorInvalidValue;
     if (p.splits > 1) {
-        launch_dtype<true>(p, a_bf16, silu, grid, plan.wm, st);
+        launch_dtype<true>(p, a_bf16, silu, grid, plan, st);
         (void)launch_splitk_reduce(p, st);
     } else {
-        launch_dtype<false>(p, a_bf16, silu, grid, plan.wm, st);
+        launch_dtype<false>(p, a_bf16, silu, grid, plan, st);
     }
     return hipGetLastError();
 }
@@ -336,7 +351,6 @@ void launch_rrn_s(const GemmParams& p, const float* norm_w, float eps, uint16_t*
                   uint16_t* norm_out, int sr, hipStream_t st) {
     const dim3 g(p.M), t(256);
     switch (p.splits) {
-    case 1: hipLaunchKernelGGL((q4_splitk_residual_rms_norm_kernel<VPT, 1>), g, t, 0, st, p, norm_w, eps, res_out, norm_out, sr); break;
     case 2: hipLaunchKernelGGL((q4_splitk_residual_rms_norm_kernel<VPT, 2>), g, t, 0, st, p, norm_w, eps, res_out, norm_out, sr); break;
     case 3: hipLaunchKernelGGL((q4_splitk_residual_rms_norm_kernel<VPT, 3>), g, t, 0, st, p, norm_w, eps, res_out, norm_out, sr); break;
     case 4: hipLaunchKernelGGL((q4_splitk_residual_rms_norm_kernel<VPT, 4>), g, t, 0, st, p, norm_w, eps, res_out, norm_out, sr); break;
@@ -344,7 +358,7 @@ void launch_rrn_s(const GemmParams& p, const float* norm_w, float eps, uint16_t*
     }
 }
 
-// GEMM into fp32 partials (one or more K splits; p.ws holds
+// GEMM into fp32 partials (gemm_splits(p) > 1; p.ws holds
 // gemm_partials_workspace_bytes(p)), then the fused reduce + residual +
 // RMSNorm pass.  Requires N % 8 == 0, N <= 16384 and 16-byte aligned rows.
 hipError_t launch_gemm_residual_rms_norm(GemmParams p, bool a_bf16, const float* norm_w, float eps,
@@ -353,7 +367,8 @@ hipError_t launch_gemm_residual_rms_norm(GemmParams p, bool a_bf16, const float*
     if (p.M <= 0 || p.N <= 0) return hipSuccess;
     if (p.N % 8 != 0 || p.N / 8 > 8 * 256 || !p.ws || !p.residual) return hipErrorInvalidValue;
     if ((long)p.M * 256 > 0xffffffffL) return hipErrorInvalidValue;   // one 256-thread block per row
-    const GemmPlan plan = plan_gemm(p, true, true);
+    const GemmPlan plan = plan_gemm(p, true);
+    if (plan.splits < 2) return hipErrorInvalidValue;
     p.nib_mask = 0x0F0F0F0Fu;
     p.tiles_m = plan.tiles_m;
     p.tiles_n = plan.tiles_n;
@@ -362,7 +377,7 @@ hipError_t launch_gemm_residual_rms_norm(GemmParams p, bool a_bf16, const float*
     const long blocks = (long)p.tiles_m * p.tiles_n * p.splits;
     const long grid = (blocks + 7) / 8 * 8;
     if (grid > 0x7fffffffL) return hipErrorInvalidValue;
-    launch_dtype<true>(p, a_bf16, false, grid, plan.wm, st);
+    launch_dtype<true>(p, a_bf16, false, grid, plan, st);
     const int vpt = (p.N / 8 + 255) / 256;
     const int sr = sum_rounded ? 1 : 0;
     if (vpt == 1)

@@ -132,6 +132,16 @@ struct SB {
 // wait counts.  GEN = true: any supported shape (K % 32 == 0, group
 // 32/64/128): scale/bias staged through registers, clamped tails, zero-filled
 // A past K, full waits.
+// KG = 2: tiles of 128 weight rows, for launches whose 256-row tiles are too
+// few.  Four waves share the rows, and the two halves of the block each take
+// two of a k-tile's four k-steps: every packed word is still dequantized once
+// and feeds BM/32 MFMAs, and the halves' sums meet in LDS after the loop.
+// Half the work between barriers makes a k-tile 0.55 us, not half of 0.95: it
+// pays only where it saves K splits or fills idle CUs (figures at the plan).
+// Measured and not kept: a ring reaching five k-tiles ahead (the same time: it
+// does not wait for copies), and waves of 64 weight rows x half of the
+// activation rows, which halve the LDS reads but dequantize every word twice
+// (M = 750, N = 5120, K = 3072: 36 us against 33.7).
 // A32: fp32 activations (the generic path only), each cast to fp16 as
 // half(clamp(x, -65504, 65504)) -- cast_f32_to_f16, Kernels.swift:816-822,
 // which DiTLinear.applyF32in runs before matmulQ4FastF32
@@ -154,19 +164,24 @@ struct SB {
 // and group 128 took 200 us, 159 here; a Llama layer at M = 96 and group 32
 // 97.4, 91.4 here.
 template <int WM, bool BF16, bool SILU, bool GEN, bool SPLIT, bool A32 = false, bool PERSIST = false,
-          int GS = 1>
+          int GS = 1, int KG = 1>
 __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
     static_assert(!A32 || (GEN && !BF16 && !SILU), "fp32 activations: the generic fp16 path");
     static_assert(!PERSIST || (!GEN && !SPLIT && !A32), "persistent tiles: the fast unsplit path");
+    static_assert(KG == 1 || (KG == 2 && !GEN && !PERSIST && WM % 2 == 0), "k-step halves: the fast single-round path");
     constexpr int BM = 64 * WM;
     constexpr int TM = BM / 32;                // MFMA tiles along M per wave
     constexpr int A_STAGE = BM * BK / 8;       // 16-byte slots per A stage
     constexpr int NA = A_STAGE / kThreads;     // A copies per thread per k-tile
-    constexpr int WP_STAGE = BN * 4;           // packed W of two k-tiles: 64 B per row
+    constexpr int BNB = BN / KG, NWN = NW / KG;    // weight rows per block, waves along them
+    constexpr int KSN = BK / 16 / KG;              // k-steps per wave and k-tile
+    constexpr int WP_STAGE = BNB * 4;          // packed W of two k-tiles: 64 B per row
     constexpr int NWP = WP_STAGE / kThreads;   // packed-W copies per thread per super-stage
-    constexpr int NPAIR = BN * GPMAX / kThreads;   // GEN: (row, group) pairs per thread per super-stage
+    constexpr int NPAIR = BNB * GPMAX / kThreads;   // GEN: (row, group) pairs per thread per super-stage
     constexpr int SBW = GS == 0 ? 4 : 2;           // fast path: scale/bias dwords per row per super-stage
-    constexpr int NSB = BN * SBW / kThreads;       // and copies of them per thread
+    // and copies of them per thread (128 rows x 2 dwords: waves 4-7 repeat
+    // the copies of waves 0-3, same bytes and slots)
+    constexpr int NSB = (BNB * SBW + kThreads - 1) / kThreads;
     // Each stage is its own array: the compiler then knows that reads of one
     // stage do not alias a direct-to-LDS copy in flight into another, and
     // does not wait for that copy (stage indices are compile-time below).
@@ -176,7 +191,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
     // of two groups (GS = 0: [k-tile][scales, biases]), copied direct to LDS.
     // Generic path: [row * GP + group] = scale | bias << 16, staged through
     // registers.
-    __shared__ uint32_t lds_sb0[GEN ? BN * GPMAX : BN * SBW], lds_sb1[GEN ? BN * GPMAX : BN * SBW];
+    __shared__ uint32_t lds_sb0[GEN ? BNB * GPMAX : BNB * SBW], lds_sb1[GEN ? BNB * GPMAX : BNB * SBW];
     static_assert(NSA == 4, "stage arrays");
     // A stage of k-tile t is t % 4, packed-W stage of super-stage ss is ss % 2.
     auto a_stage = [&](auto sc) -> u32x4* {
@@ -230,12 +245,14 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
     // m0 / n0: the tile the copies are reading (PERSIST: the next one from
     // its first prefetch on); em0 / en0: the tile the accumulators hold.
     int m0 = (tile % p.tiles_m) * BM;
-    int n0 = (tile / p.tiles_m) * (SILU ? BN / 2 : BN);
+    int n0 = (tile / p.tiles_m) * (SILU ? BNB / 2 : BNB);
     int em0 = m0, en0 = n0;
     bool has_next = PERSIST && logical + pstride < pend;
 
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wn = tid >> 6;
+    // KG = 2: wave wv owns weight rows 32 (wv % 4) .. and k-steps 2 (wv / 4) ..
+    const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = KG == 1 ? wv : wv % NWN, kg = KG == 1 ? 0 : wv / NWN;
     const int lrow = lane & 31, h = lane >> 5;
     const int GP = 4 >> p.gshift;   // scale/bias groups per 128 k (g = 32, 64, 128)
 
@@ -243,7 +260,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
     // virtual rows 32wn..32wn+31 (one 32-row MFMA tile); with SILU its rows
     // 0-15 are the gate rows and 16-31 the up rows of the same 16 output
     // columns, n0 + 16wn .. +15, so that both halves of each output land in
-    // one lane (see the epilogue).  Rows past N are clamped to row 0:
+    // one lane (see the epilogue).  Rows past N are clamped to the last row:
     // computed, never stored.
     auto wrow = [&](int v, const uint32_t*& W, const uint16_t*& S, const uint16_t*& B) {
         int n;
@@ -259,7 +276,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
             S = p.s0;
             B = p.b0;
         }
-        return n < p.N ? n : 0;
+        return n < p.N ? n : p.N - 1;
     };
 
     // ---- A: direct global -> LDS (global_load_lds_dwordx4) ----
@@ -267,18 +284,25 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
     // slot +l.  Slot s is physical column s % 8 of row s / 8, i.e. logical
     // column (s % 8) ^ xor(row): the swizzle is applied on the global side.
     // Rows past M are clamped to M-1.
-    const uint16_t* A = reinterpret_cast<const uint16_t*>(p.a);
-    const uint16_t* a_src[NA];
+    // A source is a base that is the same for the whole wave (SGPRs: the tile
+    // and the k offset) plus a byte offset per lane that no k-tile changes, so
+    // a copy needs no address arithmetic in vector registers (fast path: 32
+    // bits, K <= 2^22 keeps a tile's rows within them; 24 VGPRs fewer at 192
+    // rows, and the DiT up, lm_head and M = 333 gate/up launches 1% faster).
+    using off_t = std::conditional_t<GEN, size_t, uint32_t>;
+    constexpr int AB = A32 ? 4 : 2;   // bytes of an activation
+    const char* a_base;
+    off_t a_off[NA];
     int a_col8[NA];
     auto set_a_src = [&]() {
+        a_base = reinterpret_cast<const char*>(p.a) + ((size_t)m0 * p.K + kb * BK) * AB;
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            const int slot = (wn + NW * i) * 64 + lane;
+            const int slot = (wv + NW * i) * 64 + lane;
             const int row = slot >> 3;
             const int c16 = (slot & 7) ^ (row & 7) ^ ((row >> 3) & 1);
-            const int m = m0 + row;
             a_col8[i] = c16 * 8;
-            a_src[i] = A + (size_t)(m < p.M ? m : p.M - 1) * p.K + kb * BK + c16 * 8;
+            a_off[i] = ((off_t)(m0 + row < p.M ? row : p.M - 1 - m0) * (off_t)p.K + c16 * 8) * AB;
         }
     };
     set_a_src();
@@ -287,19 +311,24 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
     // Four lanes cover a row's 64 bytes, so each wave-wide copy reads 16 rows
     // of 64 contiguous bytes.  Slot s is row s / 4, physical piece s % 4 =
     // logical piece ^ ((row >> 2) & 3) (conflict-free reads below).
-    const uint32_t* wp_src[NWP];
+    // SILU: copy i covers virtual rows 16 (wv + NW i) .. +15, so all of a
+    // wave's copies are gate rows (even wv) or up rows (odd wv): one base.
+    const char* wp_base;
+    off_t wp_off[NWP];
     int wp_piece[NWP];
     auto set_wp_src = [&]() {
+        wp_base = reinterpret_cast<const char*>(SILU && (wv & 1) ? p.w1 : p.w0) +
+                  ((size_t)n0 * p.K + kb * BK) / 2;
 #pragma unroll
         for (int i = 0; i < NWP; ++i) {
-            const int slot = (wn + NW * i) * 64 + lane;
+            const int slot = (wv + NW * i) * 64 + lane;
             const int row = slot >> 2;
             const int piece = (slot & 3) ^ ((row >> 2) & 3);
             const uint32_t* W;
             const uint16_t *S, *B;
-            const int n = wrow(row, W, S, B);
+            const int n = wrow(row, W, S, B) - n0;
             wp_piece[i] = piece;
-            wp_src[i] = W + (size_t)n * (p.K / 8) + kb * (BK / 8) + piece * 4;
+            wp_off[i] = (off_t)n * (off_t)(p.K / 2) + piece * 16;
         }
     };
     set_wp_src();
@@ -313,11 +342,12 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
     // groups g & ~1 and g | 1, g = g_base + ss.  All are 4-byte aligned: a
     // row's groups are even in number (K % 128 == 0, GS = 2: K % 256), and so
     // is g_base for GS < 2 (splits cover whole super-stages).
+    auto sb_slot0 = [&](int i) { return (wv + NW * i) * 64 % (BNB * SBW); };
     const uint32_t* sbd_src[NSB];
     auto set_sbd_src = [&]() {
 #pragma unroll
         for (int i = 0; i < NSB; ++i) {
-            const int slot = (wn + NW * i) * 64 + lane;
+            const int slot = sb_slot0(i) + lane;
             const uint32_t* W;
             const uint16_t *S, *B;
             const int n = wrow(slot / SBW, W, S, B);
@@ -339,7 +369,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
         const int row = v / GP, g = v % GP;
         const uint32_t* W;
         const uint16_t *S, *B;
-        const int n = wrow(row < BN ? row : 0, W, S, B);
+        const int n = wrow(row < BNB ? row : 0, W, S, B);
         s_src[u] = S + (size_t)n * p.groups + g_base + g;
         b_src[u] = B + (size_t)n * p.groups + g_base + g;
         sb_g[u] = g;
@@ -350,23 +380,21 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
     // with its parity.
     // A32: this thread's eight fp32 values of each of its NA slots.
     f32x4 a32[A32 ? NA : 1][2];
-    const float* const A32src = reinterpret_cast<const float*>(p.a);
     auto load_a = [&](auto tp, int t) {   // NA (A32: 2 NA) vector-memory ops (tiles past the end re-read the last)
         const int k0 = min(t, nk - 1) * BK;
         u32x4* stage = a_stage(tp);
+        const char* base = GEN ? a_base : a_base + (size_t)k0 * AB;
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            int off = k0;
-            if (GEN && k0 + a_col8[i] >= Kl) off = Kl - 8 - a_col8[i];
+            off_t off = a_off[i];
+            if constexpr (GEN) off += (k0 + a_col8[i] >= Kl ? Kl - 8 - a_col8[i] : k0) * AB;
             if constexpr (A32) {
-                // the slot's fp16 offset in A is also its fp32 element offset
-                const f32x4* src = reinterpret_cast<const f32x4*>(
-                    A32src + (a_src[i] - reinterpret_cast<const uint16_t*>(p.a)) + off);
+                const f32x4* src = reinterpret_cast<const f32x4*>(base + off);
                 a32[i][0] = src[0];
                 a32[i][1] = src[1];
             } else {
-                __builtin_amdgcn_global_load_lds((const void*)(a_src[i] + off),
-                                                 (lds_ptr_t)(stage + (wn + NW * i) * 64), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((const void*)(base + off),
+                                                 (lds_ptr_t)(stage + (wv + NW * i) * 64), 16, 0, 0);
             }
         }
     };
@@ -386,7 +414,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
                            ((uint32_t)f2h(fminf(fmaxf(hi, -65504.0f), 65504.0f)) << 16);
                 }
                 if (k0 + a_col8[i] >= Kl) o = u32x4{0u, 0u, 0u, 0u};
-                stage[(wn + NW * i) * 64 + lane] = o;
+                stage[(wv + NW * i) * 64 + lane] = o;
             }
         }
     };
@@ -397,17 +425,19 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
         const u32x4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
         for (int i = 0; i < NA; ++i)
-            if (k0 + a_col8[i] >= Kl) stage[(wn + NW * i) * 64 + lane] = z;
+            if (k0 + a_col8[i] >= Kl) stage[(wv + NW * i) * 64 + lane] = z;
     };
     auto load_wp = [&](auto sp, int ss) {   // NWP vector-memory ops
         const int sc = min(ss, nss - 1);
         u32x4* stage = wp_stage(sp);
+        const char* base = GEN ? wp_base : wp_base + (size_t)sc * 64;   // 64 bytes per super-stage
 #pragma unroll
         for (int i = 0; i < NWP; ++i) {
-            int off = sc * 16;   // u32 words: 64 bytes per super-stage
-            if (GEN && sc * 128 + wp_piece[i] * 32 >= Kl) off = (Kl / 8) - 4 - wp_piece[i] * 4;
-            __builtin_amdgcn_global_load_lds((const void*)(wp_src[i] + off),
-                                             (lds_ptr_t)(stage + (wn + NW * i) * 64), 16, 0, 0);
+            off_t off = wp_off[i];
+            if constexpr (GEN)
+                off += sc * 128 + wp_piece[i] * 32 >= Kl ? Kl / 2 - 16 - wp_piece[i] * 16 : sc * 64;
+            __builtin_amdgcn_global_load_lds((const void*)(base + off),
+                                             (lds_ptr_t)(stage + (wv + NW * i) * 64), 16, 0, 0);
         }
     };
     auto load_sb_dma = [&](auto sp, int ss) {   // fast path: NSB vector-memory ops
@@ -417,7 +447,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
 #pragma unroll
         for (int i = 0; i < NSB; ++i)
             __builtin_amdgcn_global_load_lds((const void*)(sbd_src[i] + off),
-                                             (lds_ptr_t)(stage + (wn + NW * i) * 64), 4, 0, 0);
+                                             (lds_ptr_t)(stage + sb_slot0(i)), 4, 0, 0);
     };
     uint32_t s_reg[NPAIR], b_reg[NPAIR];
     auto load_sb = [&](int ss) {   // generic path: 2 NPAIR vector-memory ops
@@ -438,9 +468,10 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
             stage[tid + kThreads * u] = (s_reg[u] & 0xFFFFu) | (b_reg[u] << 16);
     };
 
-    // Packed words (16 bytes: this lane's four k-steps) and scale|bias of
+    // Packed words (16 bytes: this lane's k-steps; KG = 2: its half) and scale|bias of
     // tile t for both of the wave's 32-row MFMA tiles.
-    auto fetch_w = [&](auto tp, int t, u32x4 (&wk)[NT], SB& sb) {
+    typedef uint32_t wk_t __attribute__((ext_vector_type(KSN)));
+    auto fetch_w = [&](auto tp, int t, wk_t (&wk)[NT], SB& sb) {
         constexpr int TP = decltype(tp)::value & 3;
         constexpr int TL = TP & 1, SP = (TP >> 1) & 1;   // tile within / parity of super-stage
         const u32x4* ws = wp_stage(std::integral_constant<int, SP>{});
@@ -448,7 +479,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             const int vr = wn * 32 * NT + j * 32 + lrow;
-            wk[j] = ws[vr * 4 + (piece ^ ((vr >> 2) & 3))];
+            wk[j] = reinterpret_cast<const wk_t*>(ws + vr * 4 + (piece ^ ((vr >> 2) & 3)))[kg];
             uint32_t v;
             if constexpr (GEN) {
                 v = sb_stage(std::integral_constant<int, SP>{})[vr * GP + (piece >> p.gshift)];
@@ -466,7 +497,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
         }
     };
     // B fragment of k-step ks for MFMA tile j.
-    auto dequant = [&](const u32x4 (&wk)[NT], const SB& sb, int ks, u32x4 (&dst)[NT]) {
+    auto dequant = [&](const wk_t (&wk)[NT], const SB& sb, int ks, u32x4 (&dst)[NT]) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             const uint32_t v = sb.v[j];
@@ -481,7 +512,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
         }
     };
     auto read_a = [&](const u32x4* sa, int ks, u32x4 (&dst)[TM]) {
-        const int c16 = 4 * h + ks;
+        const int c16 = 4 * h + KSN * kg + ks;
 #pragma unroll
         for (int i = 0; i < TM; ++i) dst[i] = sa[swz(i * 32 + lrow, c16)];
     };
@@ -554,7 +585,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
     }
     SLTX_LDS_BARRIER();
 
-    u32x4 wk_c[NT], wk_n[NT];
+    wk_t wk_c[NT], wk_n[NT];
     SB sb_c, sb_n;
     u32x4 af[2][TM], bq[2][NT];
     fetch_w(I0{}, 0, wk_c, sb_c);
@@ -613,7 +644,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
         // also reads tile kt+1's packed words and scale/bias (used from step 3
         // on).
 #pragma unroll
-        for (int ks = 0; ks < BK / 16; ++ks) {
+        for (int ks = 0; ks < KSN; ++ks) {
             const int b = ks & 1;
 #pragma unroll
             for (int i = 0; i < TM; ++i)
@@ -621,7 +652,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
                 for (int j = 0; j < NT; ++j)
                     acc[i][j] = TRANS ? mfma32<BF16>(bq[b][j], af[b][i], acc[i][j])
                                       : mfma32<BF16>(af[b][i], bq[b][j], acc[i][j]);
-            if (ks + 1 < BK / 16) {
+            if (ks + 1 < KSN) {
                 read_a(sa, ks + 1, af[b ^ 1]);
                 dequant(wk_c, sb_c, ks + 1, bq[b ^ 1]);
             } else {
@@ -672,6 +703,33 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
         sb_c = sb_n;
     };
 
+    // ---- KG = 2: the two K halves of each tile ----
+    // Waves wv and wv + 4 hold partial sums of the same outputs.  Each gives
+    // the other half of its tiles through the idle A stages (two waves a
+    // stage) and keeps TM / 2 tiles, from tile kg TM / 2 on, in acc[0..].
+    constexpr int TMO = TM / KG;
+    auto add_k_halves = [&]() {
+        static_assert(KG == 1 || 2 * TMO * 4096 <= A_STAGE * 16, "two waves' exchange fits an A stage");
+        SLTX_WAIT_VMCNT(0);
+        SLTX_LDS_BARRIER();
+        auto buf = [&](int w) -> float* {
+            u32x4* st = (w >> 1) == 0 ? lds_a0 : (w >> 1) == 1 ? lds_a1 : (w >> 1) == 2 ? lds_a2 : lds_a3;
+            return reinterpret_cast<float*>(st) + (w & 1) * TMO * 1024 + lane;
+        };
+        float* const mine = buf(wv);
+#pragma unroll
+        for (int i = 0; i < TMO; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) mine[(i * 16 + v) * 64] = kg ? acc[i][0][v] : acc[TM - TMO + i][0][v];
+        SLTX_LDS_BARRIER();
+        const float* const other = buf(wv ^ NWN);
+#pragma unroll
+        for (int i = 0; i < TMO; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                acc[i][0][v] = (kg ? acc[TM - TMO + i][0][v] : acc[i][0][v]) + other[(i * 16 + v) * 64];
+    };
+
     // ---- epilogue, from registers (TRANS) ----
     // The MFMAs compute D^T = W_tile . A_tile^T, so lane l holds, for activation row em0 + 32 i + l % 32,
     // the wave's weight rows 8 g + 4 h + r (r = 0..3, h = l / 32) in
@@ -702,8 +760,8 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
         const bool vec = out_vec_ok(p);
         const int cw = en0 + (SILU ? 16 : 32) * wn + 8 * h;   // this lane's first column
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const int m = em0 + i * 32 + lrow;   // lanes l and l + 32 share a row
+        for (int i = 0; i < TMO; ++i) {
+            const int m = em0 + (kg * TMO + i) * 32 + lrow;   // lanes l and l + 32 share a row
             float x[8];
             if constexpr (SPLIT) {
                 // raw fp32 partial sums; the reduce kernel applies the epilogue
@@ -756,37 +814,37 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
         SLTX_LDS_BARRIER();
         float* const eb0 = reinterpret_cast<float*>(lds_a0);
         float* const eb1 = reinterpret_cast<float*>(lds_a1);
-        float* const wdst = (wn >> 2) ? eb1 : eb0;
+        // KG = 2: the second buffer holds the other K half's tile (128 columns)
+        float* const wdst = (wv >> 2) ? eb1 : eb0;
         const int wcol = (wn & 3) * 32 + lrow;
         const int er = tid >> 4, ec = (tid & 15) * 8;
         const bool vec = out_vec_ok(p);
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
+        for (int i = 0; i < TMO; ++i) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) wdst[(8 * (v >> 2) + 4 * h + (v & 3)) * 128 + wcol] = acc[i][0][v];
             SLTX_LDS_BARRIER();
             const int m = em0 + i * 32 + er;
-            if (m < p.M) {
-                float x0[8], x1[8];
-                const f32x4* r0 = reinterpret_cast<const f32x4*>(eb0 + er * 128 + ec);
-                const f32x4* r1 = reinterpret_cast<const f32x4*>(eb1 + er * 128 + ec);
-                const f32x4 a0 = r0[0], a1 = r0[1], b0 = r1[0], b1 = r1[1];
+            // eb1's rows and columns
+            const int m1 = KG == 1 ? m : m + TMO * 32, c1 = KG == 1 ? en0 + 128 + ec : en0 + ec;
+            float x0[8], x1[8];
+            const f32x4* r0 = reinterpret_cast<const f32x4*>(eb0 + er * 128 + ec);
+            const f32x4* r1 = reinterpret_cast<const f32x4*>(eb1 + er * 128 + ec);
+            const f32x4 a0 = r0[0], a1 = r0[1], b0 = r1[0], b1 = r1[1];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    x0[e] = a0[e];
-                    x0[4 + e] = a1[e];
-                    x1[e] = b0[e];
-                    x1[4 + e] = b1[e];
-                }
-                if constexpr (SPLIT) {
-                    // raw fp32 partial sums; the reduce kernel applies the epilogue
-                    float* wsr = p.ws + ((size_t)split * p.M + m) * (size_t)p.N;
-                    store_f32x8(wsr, en0 + ec, p.N, x0);
-                    store_f32x8(wsr, en0 + 128 + ec, p.N, x1);
-                } else {
-                    epi_store8(p, (size_t)m * p.N, en0 + ec, x0, vec);
-                    epi_store8(p, (size_t)m * p.N, en0 + 128 + ec, x1, vec);
-                }
+            for (int e = 0; e < 4; ++e) {
+                x0[e] = a0[e];
+                x0[4 + e] = a1[e];
+                x1[e] = b0[e];
+                x1[4 + e] = b1[e];
+            }
+            if constexpr (SPLIT) {
+                // raw fp32 partial sums; the reduce kernel applies the epilogue
+                if (m < p.M) store_f32x8(p.ws + ((size_t)split * p.M + m) * (size_t)p.N, en0 + ec, p.N, x0);
+                if (m1 < p.M) store_f32x8(p.ws + ((size_t)split * p.M + m1) * (size_t)p.N, c1, p.N, x1);
+            } else {
+                if (m < p.M) epi_store8(p, (size_t)m * p.N, en0 + ec, x0, vec);
+                if (m1 < p.M) epi_store8(p, (size_t)m1 * p.N, c1, x1, vec);
             }
             SLTX_LDS_BARRIER();
         }
@@ -805,6 +863,7 @@ __global__ __launch_bounds__(kThreads, 1) void q4_gemm_kernel(GemmParams p) {
             if (kt + 1 < nk) step(I1{}, kt + 1);
             if (kt + 2 < nk) step(I2{}, kt + 2);
         }
+        if constexpr (KG == 2) add_k_halves();
         if constexpr (PERSIST || SILU) {
             // the block's last copies (clamped re-reads of the last k-tile)
             // land before it ends and its LDS is released; the stores need

@@ -225,10 +225,11 @@ size_t gemm_workspace_bytes(const GemmParams& p);
 // Launches the GEMM; splits K only if p.ws is non-null (and then needs
 // gemm_workspace_bytes(p) bytes there).
 hipError_t launch_gemm(GemmParams p, bool a_bf16, hipStream_t st);
-// Bytes of fp32 partials the fused residual + RMSNorm GEMM of `p` uses (its
-// output always goes through the workspace, at one split or more).
+// K splits of the GEMM's plan for p, and the bytes of fp32 partials they take
+// (counted for one split too).
+int gemm_splits(const GemmParams& p);
 size_t gemm_partials_workspace_bytes(const GemmParams& p);
-// GEMM (no epilogue; p.residual is the residual input) into the workspace
+// GEMM of more than one K split (no epilogue; p.residual is the residual input) into the workspace
 // p.ws, then one pass per row: res_out = half(residual + half(sum of splits))
 // and norm_out = rms_norm(res_out) with the sum of squares over the unrounded
 // sum (sum_rounded false) or over res_out (true).  N % 8 == 0, N <= 16384.

@@ -1,7 +1,11 @@
 """The GEMM's fast kernel at group sizes 32 and 128 (scale / bias dwords copied
-direct to LDS) against its generic kernel, which stages them through registers
-and which a scale array at an odd 2-byte address selects: the same plan, k
-order and dequantization, so the results must be equal bit for bit.  The
+direct to LDS) and both its weight-tile widths against its generic kernel,
+which stages them through registers and which a scale array at an odd 2-byte
+address selects.  Both dequantize alike; K splits and the halves of the
+128-row weight tiles may add the fp32 sums in another order.  An output is
+K / 16 MFMA steps, each rounding a partial sum of at most about the largest
+output once, on either side: the difference is bounded by
+2 (K / 16) 2^-24 max|y| (fp16 outputs: one more half ulp on either side).  The
 generic kernel is held to the oracle in test_gpu_gemm.py; one case here is too.
 
 K covers one and several super-stages (128 k), odd counts of them, and at
@@ -26,9 +30,17 @@ def _odd(t):
     return v
 
 
+def _close(a, b, K, half=False):
+    a, b = a.double(), b.double()
+    tol = 2 * (K / 16) * 2.0**-24 * b.abs().max() + (2.0**-10 * b.abs() if half else 0.0)
+    return bool(((a - b).abs() <= tol).all())
+
+
 # (300, 500, 1280) splits K; (1000, 16384, 512) runs persistent blocks
 SHAPES = [(257, 256, 256), (300, 500, 1280), (300, 777, 3328), (513, 3072, 3072), (700, 1000, 768),
-          (1000, 16384, 512)]
+          (1000, 16384, 512),
+          # 128-row weight tiles: one round, partial tiles; three K splits (bf16)
+          (700, 5000, 1280), (1537, 2040, 2304), (300, 2048, 2560)]
 
 
 @pytest.mark.parametrize("g", [32, 64, 128])
@@ -40,11 +52,11 @@ def test_fast_equals_generic(pkg, dev, M, N, K, g):
         fast = pkg.matmul_q4_ex(x, pkg.Q4Weight(w, s, b, K, g), M, N)
         gen = pkg.matmul_q4_ex(x, pkg.Q4Weight(w, _odd(s), _odd(b), K, g), M, N)
         torch.cuda.synchronize()
-        assert torch.equal(fast, gen), f"{dt} M={M} N={N} K={K} g={g}"
+        assert _close(fast, gen, K), f"{dt} M={M} N={N} K={K} g={g}"
 
 
 @pytest.mark.parametrize("g", [32, 128])
-@pytest.mark.parametrize("M,N,K", [(300, 200, 512), (700, 8192, 768), (500, 384, 3072)])
+@pytest.mark.parametrize("M,N,K", [(300, 200, 512), (700, 8192, 768), (500, 384, 3072), (200, 8000, 1280)])
 def test_fast_equals_generic_pair(pkg, dev, M, N, K, g):
     import torch
     x, sets = gpu_inputs(M, N, K, g, seed=M + K, dev=dev, n_weights=2)
@@ -52,7 +64,7 @@ def test_fast_equals_generic_pair(pkg, dev, M, N, K, g):
     gen = pkg.matmul_q4_silu_mul(x, *(pkg.Q4Weight(w, _odd(s), _odd(b), K, g) for w, s, b in sets),
                                  M, K, N)
     torch.cuda.synchronize()
-    assert torch.equal(fast, gen)
+    assert _close(fast, gen, K, half=True)
 
 
 @pytest.mark.parametrize("g", [32, 128])
