@@ -343,7 +343,8 @@ int sltx_sample_top_p_state(const void* logits, int32_t dtype, int32_t n, float 
  * launched and no device is needed.  Returns an sltx_route, or a negative
  * sltx_status for invalid arguments. */
 typedef enum {
-    SLTX_ROUTE_GEMM = 0,     /* MFMA GEMM, split over K when its tiles would not fill the GPU */
+    SLTX_ROUTE_GEMM = 0,     /* MFMA GEMM, split over K when its tiles would not fill the GPU (fp32 x
+                                of few columns: its strip kernel, which casts x in registers) */
     SLTX_ROUTE_SMALL_M = 1,  /* small-M weight stream (M <= 32, 16x16x32 MFMA) */
     SLTX_ROUTE_NARROW = 2,   /* narrow weight stream (one weight set, M <= 4, 4x4x4 MFMA) */
     SLTX_ROUTE_MID = 3,      /* pipelined weight stream (8 < M <= 32, from M = 6 for a set of at most

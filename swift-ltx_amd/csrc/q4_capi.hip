@@ -370,6 +370,7 @@ int run_gemm(const char* fn, const void* x, int x_dtype, const sltx_q4_weight& w
         }
         return finish(launch_wide(p, wp, st), fn);
     }
+    if (strip_ok(p)) return finish(launch_strip(p, st), fn);
     const size_t need = gemm_workspace_bytes(p);
     if (need > 0) p.ws = stream_workspace(st, need);
     return finish(launch_gemm(p, x_dtype == kBF16, st), fn);

@@ -220,6 +220,11 @@ hipError_t launch_wide(GemmParams p, const WidePlan& pl, hipStream_t st);
 // The split-K reduce pass: y = epilogue(sum of p.splits fp32 partials in p.ws).
 hipError_t launch_splitk_reduce(const GemmParams& p, hipStream_t st);
 
+// fp32 x and few output columns (q4_strip.hip): the GEMM family's kernel where
+// strip_ok.
+bool strip_ok(const GemmParams& p);
+hipError_t launch_strip(GemmParams p, hipStream_t st);
+
 // Bytes of split-K workspace the launch of `p` would use (0: it does not split).
 size_t gemm_workspace_bytes(const GemmParams& p);
 // Launches the GEMM; splits K only if p.ws is non-null (and then needs

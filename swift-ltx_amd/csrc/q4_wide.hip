@@ -36,19 +36,17 @@
 //    arrive adds the splits in split order and runs the epilogue (no reduce
 //    pass).
 #include <type_traits>
-#include <utility>
 
 #include "q4_common.hpp"
 #include "q4_dequant.hpp"
 #include "q4_epilogue.hpp"
 #include "q4_launch.hpp"
+#include "q4_ring.hpp"
 #include "q4_split.hpp"
 
 namespace sltx {
 
 namespace {
-
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 constexpr int NWV = 8;              // waves, one K-group each
 constexpr int WT = 64 * NWV;        // threads per block
@@ -70,48 +68,10 @@ constexpr int SLAB_G = 128;         // scale / bias groups a block holds
 template <int TM>
 constexpr int wide_nsx() { return TM == 4 ? 3 : 4; }
 
-#define WIDE_LDS_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
-
-// f(integral_constant<int, i>) for i = 0 .. N - 1, unrolled
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_seq(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_seq(f, std::make_integer_sequence<int, N>{});
-}
-
 struct WideArgs {
     int mrows;    // activation rows of this launch's M-blocks (the last may hold fewer)
     int kblk;     // k per split
 };
-
-// LDS reads the compiler does not see as memory operations.  Its wait-count
-// pass cannot tell reads of one ring stage from copies in flight into
-// another once the loop's back-edge merges its state, and would drain every
-// copy in flight (vmcnt(0)) before the first read of each unrolled
-// iteration; the stage a round reads has been waited for by that round's
-// own vmcnt and barrier.  The results must pass through lds_wait() before
-// use.
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-    return (uint32_t)(uintptr_t)(lds_ptr_t)(p);
-}
-__device__ __forceinline__ u32x4 ds_read16(uint32_t a) {
-    u32x4 v;
-    asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(a) : "memory");
-    return v;
-}
-__device__ __forceinline__ uint32_t ds_read4(uint32_t a) {
-    uint32_t v;
-    asm volatile("ds_read_b32 %0, %1" : "=v"(v) : "v"(a) : "memory");
-    return v;
-}
-
-__device__ __forceinline__ f32x16 mfma32_f16(u32x4 a, u32x4 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
 
 // X piece (row, c) of a stage sits at row * XCH + (c ^ (row & 15)): the 16
 // rows a quarter-wave reads at one logical piece hit 16 distinct pieces.
@@ -398,7 +358,7 @@ __global__ __launch_bounds__(WT, 1) void q4_wide_kernel(GemmParams p, WideArgs w
             __builtin_amdgcn_s_waitcnt(vmcnt_only((NSX - 2) * CPR_W));
         else
             __builtin_amdgcn_s_waitcnt(vmcnt_only((NSX - 2) * CPR_X));
-        WIDE_LDS_BARRIER();
+        RING_LDS_BARRIER();
     };
     // Round q (operands in a, b): round q + 1's stage is waited for, the
     // stage round q read is refilled with round q + NSX, round q + 1's LDS
@@ -446,7 +406,7 @@ __global__ __launch_bounds__(WT, 1) void q4_wide_kernel(GemmParams p, WideArgs w
     // over the 8 waves, in wave order.
     constexpr int G = XS * 16 >= 2 * 2 * 8 * 1024 ? 2 : 1;
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-    WIDE_LDS_BARRIER();
+    RING_LDS_BARRIER();
     auto buf = [&](int w, int d) -> float* {
         u32x4* st = (w >> 1) == 0 ? xs0 : (w >> 1) == 1 ? xs1 : (w >> 1) == 2 ? xs2
                     : NSX > 3 ? xs3 : reinterpret_cast<u32x4*>(slab);
@@ -468,7 +428,7 @@ __global__ __launch_bounds__(WT, 1) void q4_wide_kernel(GemmParams p, WideArgs w
         for (int e = 0; e < NV; ++e) own0[i][e] = own1[i][e] = 0.0f;
 #pragma unroll
     for (int i0 = 0; i0 < TM; i0 += G) {
-        if (i0 > 0) WIDE_LDS_BARRIER();
+        if (i0 > 0) RING_LDS_BARRIER();
 #pragma unroll
         for (int d = 0; d < G && i0 + d < TM; ++d) {
             float* const mine = buf(wave, d);
@@ -477,7 +437,7 @@ __global__ __launch_bounds__(WT, 1) void q4_wide_kernel(GemmParams p, WideArgs w
 #pragma unroll
                 for (int e = 0; e < 16; ++e) mine[j * 1024 + e * 64 + lane] = acc[i0 + d][j][e];
         }
-        WIDE_LDS_BARRIER();
+        RING_LDS_BARRIER();
 #pragma unroll
         for (int d = 0; d < G && i0 + d < TM; ++d) {
             const int i = i0 + d;
