@@ -131,11 +131,11 @@ struct SampleParams {
     float* probs;           // [n] scaled logits, then probabilities
     float* mpart;           // block maxima
     float* spart;           // block exp-sums (relative to the block maxima)
-    uint32_t* h0cnt;        // level-0 histogram (4096 bins)
+    uint32_t* h0cnt;        // level-0 histogram
     unsigned long long* h0mass;
     uint32_t* h0min;        // smallest and largest key (probability bits) of each
     uint32_t* h0max;        // level-0 bin: a bin of equal keys is all tied
-    uint32_t* h1cnt;        // range histogram (4096 buckets), same fields
+    uint32_t* h1cnt;        // range histogram, same fields
     unsigned long long* h1mass;
     uint32_t* h1min;
     uint32_t* h1max;

@@ -28,7 +28,7 @@
 //                   marked in an LDS bitmap); block max and exp-sum; clears
 //                   the level-0 and range histograms
 //   sample_prob     p = exp(l - max) / sum; level-0 histogram (p bits
-//                   31..20: count and mass per bin)
+//                   29..20: count and mass per bin)
 //   sample_gather   each block finds, from the histogram, the bin holding the
 //                   cutoff and the bins the draw can reach; if their untied
 //                   tokens fit the select kernel's LDS it compacts them
@@ -39,7 +39,7 @@
 //                   found by rank, from counts of the tied key per 1024-token
 //                   chunk kept during compaction.  (No grid-wide fence or
 //                   last-block hand-off: on a chip whose XCDs have separate
-//                   L2s those cost more than re-reading the 48 KB histogram
+//                   L2s those cost more than re-reading the 20 KB histogram
 //                   per block.)
 //   sample_narrow   mode 1: the same from the range histogram, compacting
 //                   the untied tokens of the buckets that matter
@@ -60,7 +60,14 @@ namespace {
 constexpr int kGridThreads = 256;   // grid kernels: 4 consecutive tokens a thread per step
 constexpr int kMaxBlocks = 256;
 constexpr int kSelThreads = 1024;   // sample_select
-constexpr int kBins = 4096;         // 12-bit digits
+// Buckets of the level-0 and range histograms.  A probability is at most 1, so
+// its key's top 12 bits are at most 0x3F8: 1024 bins hold every finite input,
+// and the last one also takes all higher keys (p NaN).  4096 bins, one for each
+// value of the 12 bits, made every block zero, merge and re-read four times as
+// much.  Measured at 128256 tokens, all five launches: peaked logits 33.4 us
+// with 4096 bins, 26.6 with 1024; all equal 38.2 / 32.4; near-flat 56.0 / 48.1.
+constexpr int kBins = 1024;
+constexpr int kLevelBins = 4096;    // the select kernel's levels: 12-bit digits
 constexpr int kCandLds = 8192;      // candidates sample_select holds in LDS
 constexpr int kSelUnroll = 8;      // candidates each select thread loads before using them
 constexpr int kNthUnroll = 16;     // 16-byte key loads a lane has in flight in nth_with_key
@@ -225,8 +232,11 @@ __device__ __forceinline__ void key_minmax(bool ok, int d, uint32_t key, int lea
     }
 }
 
-// The buckets the select positions are found in.  Mode 0: level-0 bins,
-// key >> 20.  Mode 1 (the range histogram): segment A, keys [a_lo, a_end) in
+// The level-0 bin of a key.
+__device__ __forceinline__ int level0_bin(uint32_t key) { return min((int)(key >> 20), kBins - 1); }
+
+// The buckets the select positions are found in.  Mode 0: level-0 bins.
+// Mode 1 (the range histogram): segment A, keys [a_lo, a_end) in
 // buckets [0, kSplit) of 2^a_shift keys counted from a_base; segment B, keys
 // [b_lo, b_end) in buckets [kSplit, kBins) of 2^b_shift keys counted from
 // b_base (each base is its low key rounded down to the bucket width); the
@@ -247,18 +257,20 @@ struct Buckets {
 
     // bucket of a key, kBins if none
     __device__ int of(uint32_t key) const {
-        if (!ranged) return (int)(key >> 20);
+        if (!ranged) return level0_bin(key);
         if (key >= a_lo && (unsigned long long)key < a_end) return (int)((key - a_base) >> a_shift);
         if (key >= b_lo && (unsigned long long)key < b_end)
             return kSplit + (int)((key - b_base) >> b_shift);
         return kBins;
     }
-    // bits of the order key D below bucket b's key prefix, and that prefix
+    // bits of the order key D below bucket b's key prefix, and that prefix.
+    // The last level-0 bin has none: where it holds a token the input is not
+    // finite, every p is NaN and so every token is in it.
     __device__ int low_bits(int b) const {
-        return !ranged ? 44 : (b < kSplit ? a_shift : b_shift) + 24;
+        return !ranged ? (b == kBins - 1 ? 56 : 44) : (b < kSplit ? a_shift : b_shift) + 24;
     }
     __device__ unsigned long long prefix(int b) const {
-        if (!ranged) return (unsigned long long)b << 44;
+        if (!ranged) return b == kBins - 1 ? 0ull : (unsigned long long)b << 44;
         if (b < kSplit)
             return (unsigned long long)((a_base >> a_shift) + (uint32_t)b) << (a_shift + 24);
         return (unsigned long long)((b_base >> b_shift) + (uint32_t)(b - kSplit)) << (b_shift + 24);
@@ -277,10 +289,10 @@ __device__ __forceinline__ Buckets range_buckets(const SampleParams& p, const Sa
 
 // The narrowest power-of-two bucket width (its log2) that puts the keys
 // [lo, hi] into kSegBuckets buckets counted from lo rounded down to the
-// width.  A segment has kSplit buckets; using fewer keeps the gather
-// kernel's histogram merge short (one set of device atomics per non-empty
-// bucket and block) while its buckets stay far narrower than a level-0 bin.
-constexpr uint32_t kSegBuckets = 512;
+// width: few enough to keep the gather kernel's histogram merge short (one set
+// of device atomics per non-empty bucket and block), far narrower than a
+// level-0 bin.
+constexpr uint32_t kSegBuckets = kSplit;
 
 __device__ __forceinline__ int seg_shift(uint32_t lo, uint32_t hi) {
     int sh = 0;
@@ -375,15 +387,15 @@ struct SelScratch {
     unsigned long long rem;    // nth_in_chunks: rank left; select_in_bin: inclusive mass
 };
 
-// kBins buckets in descending order, after `above` mass, spread over the
+// NB buckets in descending order, after `above` mass, spread over the
 // block (BPT consecutive buckets a thread).  load() reads the buckets and
 // scans their masses; find(target) gives the highest non-empty bucket whose
 // inclusive running mass reaches target (found), its exclusive / inclusive
 // mass and count, and the total.  Whole block; cnt and mass may be global or
 // LDS.  Both end synchronised.
-template <int NT>
+template <int NT, int NB = kBins>
 struct BinScan {
-    static constexpr int BPT = kBins / NT;
+    static constexpr int BPT = NB / NT;
     uint32_t c[BPT];
     unsigned long long m[BPT];
     uint32_t kmn[BPT], kmx[BPT];   // load_tied: each bucket's smallest and largest key
@@ -392,7 +404,7 @@ struct BinScan {
 
     __device__ void load(const uint32_t* cnt, const unsigned long long* mass,
                          unsigned long long above, SelScratch& sc) {
-        top = kBins - 1 - (int)threadIdx.x * BPT;
+        top = NB - 1 - (int)threadIdx.x * BPT;
         tot = 0ull;
 #pragma unroll
         for (int k = 0; k < BPT; ++k) {
@@ -404,11 +416,11 @@ struct BinScan {
     }
 
     // load() over a histogram with key extremes: also marks the tied buckets
-    // in tied_bm (kBins bits, LDS; written whole), and in mode 1 adds the
+    // in tied_bm (NB bits, LDS; written whole), and in mode 1 adds the
     // mass between the segments to segment A's running mass.
     __device__ void load_tied(const Buckets& bk, unsigned long long above, SelScratch& sc,
                               uint32_t* tied_bm) {
-        top = kBins - 1 - (int)threadIdx.x * BPT;
+        top = NB - 1 - (int)threadIdx.x * BPT;
         tot = 0ull;
 #pragma unroll
         for (int k = 0; k < BPT; ++k) {
@@ -472,9 +484,9 @@ struct BinScan {
 };
 
 struct LevelHist {
-    uint32_t cnt[kBins];
-    unsigned long long mass[kBins];
-    uint32_t id[kBins];
+    uint32_t cnt[kLevelBins];
+    unsigned long long mass[kLevelBins];
+    uint32_t id[kLevelBins];
 };
 
 // Calls f(c, e) for every candidate index c < C (e = cand[c]) in a
@@ -520,7 +532,7 @@ __device__ int select_in_bin(const uint2* cand, int C, const Buckets& bk, int bu
         const int shift = pos > width ? pos - width : 0;
         const unsigned long long wmask = (1ull << (pos - shift)) - 1ull;
         pos = shift;
-        for (int b = tid; b < (small ? 256 : kBins); b += kSelThreads) {
+        for (int b = tid; b < (small ? 256 : kLevelBins); b += kSelThreads) {
             H.cnt[b] = 0u;
             H.mass[b] = 0ull;
         }
@@ -570,7 +582,7 @@ __device__ int select_in_bin(const uint2* cand, int C, const Buckets& bk, int bu
             }
             __syncthreads();
         } else {
-            BinScan<kSelThreads> scan;
+            BinScan<kSelThreads, kLevelBins> scan;
             scan.load(H.cnt, H.mass, above, sc);
             scan.find(target, bs, sc);
         }
@@ -725,7 +737,8 @@ __global__ __launch_bounds__(kGridThreads) void argmax_final_kernel(const void* 
 // q = 256 b + t + k T (tokens 4q..4q+3), k = 0, 1, ...; the block's seen ids
 // are marked in an LDS bitmap indexed by (k, t, token within the quad).
 __global__ __launch_bounds__(kGridThreads) void sample_scale_kernel(SampleParams p) {
-    __shared__ float red[kGridThreads];
+    __shared__ float red[kGridThreads], wmax[kGridThreads / 64];
+    static_assert(kGridThreads == 256, "the trees below");
     __shared__ uint32_t seen_bm[kSeenWords];
     const int n = p.n;
     const int T = gridDim.x * kGridThreads;
@@ -773,14 +786,13 @@ __global__ __launch_bounds__(kGridThreads) void sample_scale_kernel(SampleParams
             mx = fmaxf(mx, l);
         }
     }
-    red[threadIdx.x] = mx;
+    // The block's max (exact in any order).  Shuffles instead of eight LDS rounds
+    // with a barrier each, here and in the sum: 0.4 - 0.7 us a call, to 26.1
+    // peaked and 47.4 near-flat at 128256 tokens.
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
     __syncthreads();
-    for (int s2 = kGridThreads / 2; s2 > 0; s2 >>= 1) {
-        if ((int)threadIdx.x < s2) red[threadIdx.x] = fmaxf(red[threadIdx.x], red[threadIdx.x + s2]);
-        __syncthreads();
-    }
-    const float mb = red[0];
-    __syncthreads();
+    const float mb = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
     float sm = 0.0f;
     for (int q = blockIdx.x * kGridThreads + threadIdx.x, kk = 0; q < nq; q += T, ++kk) {
 #pragma unroll
@@ -790,15 +802,17 @@ __global__ __launch_bounds__(kGridThreads) void sample_scale_kernel(SampleParams
             sm += expf((kk == 0 ? l0[e] : p.probs[i]) - mb);
         }
     }
+    // the halving tree: 128 and 64 apart through LDS, then within wave 0
     red[threadIdx.x] = sm;
     __syncthreads();
-    for (int s2 = kGridThreads / 2; s2 > 0; s2 >>= 1) {
-        if ((int)threadIdx.x < s2) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + s2];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        p.mpart[blockIdx.x] = mb;
-        p.spart[blockIdx.x] = red[0];
+    if (threadIdx.x < 64) {
+        const int t = threadIdx.x;
+        float v = (red[t] + red[t + 128]) + (red[t + 64] + red[t + 192]);
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+        if (t == 0) {
+            p.mpart[blockIdx.x] = mb;
+            p.spart[blockIdx.x] = v;
+        }
     }
 }
 
@@ -862,7 +876,7 @@ __global__ __launch_bounds__(kGridThreads) void sample_prob_kernel(SampleParams 
                 p.probs[i] = pv;
             }
             const uint32_t key = __float_as_uint(pv);
-            const int d = (int)(key >> 20);
+            const int d = level0_bin(key);
             const int lead = hist_add(ok, d, key, ok ? mass_of(key) : 0ull, hc, hm);
             key_minmax(ok, d, key, lead, hlo, hhi);
         }
@@ -1029,7 +1043,7 @@ __device__ void compact(const SampleParams& p, const uint32_t (&key0)[4], Want w
 // histogram over the keys of those bins (segment A: the cutoff's bin,
 // segment B: the draw's bins), which the select kernel's blocks then narrow
 // and compact.  No grid-wide fence or last-block hand-off here: on a chip
-// whose XCDs have separate L2s those cost more than re-reading the 48 KB
+// whose XCDs have separate L2s those cost more than re-reading the 20 KB
 // histogram per block.
 __global__ __launch_bounds__(kGridThreads) void sample_gather_kernel(SampleParams p) {
     constexpr int kWaves = kGridThreads / 64;
@@ -1101,7 +1115,7 @@ __global__ __launch_bounds__(kGridThreads) void sample_gather_kernel(SampleParam
             if (threadIdx.x == 0) p.ctl->ntied = nt;
             if ((int)threadIdx.x < nt) p.ctl->tkey[threadIdx.x] = s_tkey[threadIdx.x];
         }
-        compact<kGridThreads>(p, key0, [&](uint32_t key) { return want((int)(key >> 20)); },
+        compact<kGridThreads>(p, key0, [&](uint32_t key) { return want(level0_bin(key)); },
                               s_tkey, nt, offs, tsum);
         return;
     }
@@ -1515,9 +1529,10 @@ size_t argmax_workspace_bytes() { return 2 * kMaxBlocks * 4; }
 // probabilities, block maxima and exp-sums, the level-0 and range
 // histograms (count, mass, key min and max), the control block, the tied-key
 // chunk counts, candidates
+constexpr size_t kHistBytes = 20 * kLevelBins;   // more than a histogram takes (20 kBins)
 constexpr size_t sample_ws_bytes(size_t n) {
     return (n * 4 + 255) / 256 * 256 + 2 * ((kMaxBlocks * 4 + 255) / 256 * 256) +
-           2 * (3 * ((kBins * 4 + 255) / 256 * 256) + (kBins * 8 + 255) / 256 * 256) + 256 +
+           2 * kHistBytes + 256 +
            (kTiedSlots * 4 * ((n + 1023) / 1024) + 255) / 256 * 256 + (n * 8 + 255) / 256 * 256;
 }
 
@@ -1578,22 +1593,15 @@ hipError_t launch_sample(SampleParams p, void* ws, hipStream_t st) {
     w += up256(kMaxBlocks * 4);
     p.spart = reinterpret_cast<float*>(w);
     w += up256(kMaxBlocks * 4);
-    p.h0cnt = reinterpret_cast<uint32_t*>(w);
-    w += up256(kBins * 4);
-    p.h0mass = reinterpret_cast<unsigned long long*>(w);
-    w += up256(kBins * 8);
-    p.h0min = reinterpret_cast<uint32_t*>(w);
-    w += up256(kBins * 4);
-    p.h0max = reinterpret_cast<uint32_t*>(w);
-    w += up256(kBins * 4);
-    p.h1cnt = reinterpret_cast<uint32_t*>(w);
-    w += up256(kBins * 4);
-    p.h1mass = reinterpret_cast<unsigned long long*>(w);
-    w += up256(kBins * 8);
-    p.h1min = reinterpret_cast<uint32_t*>(w);
-    w += up256(kBins * 4);
-    p.h1max = reinterpret_cast<uint32_t*>(w);
-    w += up256(kBins * 4);
+    auto hist = [&](uint32_t*& cnt, unsigned long long*& mass, uint32_t*& lo, uint32_t*& hi) {
+        mass = reinterpret_cast<unsigned long long*>(w);
+        cnt = reinterpret_cast<uint32_t*>(mass + kBins);
+        lo = cnt + kBins;
+        hi = lo + kBins;
+        w += kHistBytes;
+    };
+    hist(p.h0cnt, p.h0mass, p.h0min, p.h0max);
+    hist(p.h1cnt, p.h1mass, p.h1min, p.h1max);
     static_assert(sizeof(SampleCtl) <= 256, "control block");
     p.ctl = reinterpret_cast<SampleCtl*>(w);
     w += 256;
