@@ -268,7 +268,10 @@ int release_workspace(hipStream_t st) {
 // The route run_gemm takes for p (SLTX_ROUTE_*), and the plans it launches
 // with.  One weight set at M <= 4: the narrow route (4x4x4 MFMA blocks,
 // whole-line loads), unless the small-M route runs two row tiles per block
-// at two blocks per CU (tall matrices such as the vocabulary head).
+// at two blocks per CU and K <= 3072 (tall matrices such as the vocabulary
+// head; at K = 4096 the narrow route is the faster one for 12000 rows, 9.8 -
+// 10.5 us against 10.5 - 11.0 at M = 2..4, the slower for 16384, 12.8 against
+// 11.5 - 11.9).
 // Measured on the Llama, T5 and vocabulary-head shapes at M = 2, 4, 8, that
 // is the faster route in every case; gated pairs and M > 4 are faster on the
 // small-M route, up to M = 16.
@@ -286,7 +289,7 @@ int gemm_route(const GemmParams& p, bool a_bf16, NarrowPlan* np, SkinnyPlan* sp,
     if (p.M > 32) return wide_plan(p, a_bf16, wp) ? SLTX_ROUTE_WIDE : SLTX_ROUTE_GEMM;
     const bool narrow = narrow_plan(p, a_bf16, np);
     const bool skinny = skinny_plan(p, a_bf16, sp);
-    if (narrow && (!skinny || !(sp->RT == 2 && sp->OCC == 2))) return SLTX_ROUTE_NARROW;
+    if (narrow && (!skinny || !(sp->RT == 2 && sp->OCC == 2 && p.K <= 3072))) return SLTX_ROUTE_NARROW;
     // The mid-M route: above 16 rows where it is built (at K > 3072 only
     // where the small-M route cannot run or above 24 rows), and one weight
     // set of 4096..16384 rows at K <= 3072 above 8 rows.  Measured (us per

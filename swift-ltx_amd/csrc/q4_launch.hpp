@@ -89,8 +89,8 @@ struct EmbedParams {
 // and the gather kernel compacted the candidates; mode 1: the candidate bins
 // held too many tokens, and a range histogram splits them into finer
 // buckets -- segment A, the keys [a_lo, a_end) of the cutoff's bin in
-// buckets [0, 2048) of 2^a_shift keys counted from a_base, and segment B,
-// the keys [b_lo, b_end) of the draw's bins above it in buckets [2048, 4096)
+// buckets [0, 512) of 2^a_shift keys counted from a_base, and segment B,
+// the keys [b_lo, b_end) of the draw's bins above it in buckets [512, 1024)
 // counted from b_base; each segment's range is the smallest to the largest
 // key its bins hold, and each base is its low key rounded down to the bucket
 // width.  Tied buckets (one key) get per-chunk counts of their key (up to 4:
@@ -178,10 +178,15 @@ hipError_t launch_narrow(const GemmParams& p, const NarrowPlan& pl, hipStream_t 
 // each, MT tiles of 16 activation rows, RT tiles of 16 weight rows per block.
 // skinny_plan returns false when the shape or epilogue is not covered (the
 // GEMM then runs).
+enum SkinnyX : int {
+    kXRegs = 0,   // fragments of 16 rows per tile, loaded to registers
+    kXLds = 1,    // the block's rows staged in LDS (one 16-row tile, rows that fit)
+    kXHalf = 2,   // as kXRegs for at most 8 rows: one load fills two fragments
+};
 struct SkinnyPlan {
     int W, MT, STEPS, RT;
     int OCC;   // blocks per CU the configuration is compiled for
-    bool XL;   // X staged in LDS (one 16-row tile, M * K * 2 bytes that fit)
+    int XM;    // where the waves take X from (SkinnyX)
 };
 bool skinny_plan(const GemmParams& p, bool a_bf16, SkinnyPlan* out);
 hipError_t launch_skinny(const GemmParams& p, const SkinnyPlan& pl, hipStream_t st);

@@ -19,16 +19,24 @@
 //  * The block's scales and biases (one contiguous slab per array) are
 //    copied to LDS with direct 16-byte global -> LDS loads, issued first.
 //  * The wave's slice of X (all M rows, 16 per MFMA tile) stays in
-//    registers for the whole kernel.  With one 16-row tile and M * K * 2
-//    bytes that fit (XL), the block first copies the M real rows to LDS
-//    (rows padded by 16 bytes: the 16 rows of a fragment read hit distinct
-//    banks), before its weight loads, and each wave reads its fragments from
-//    there, with zeros for rows past M: every 16-byte load through the
-//    vector memory path costs that path 16 cycles whatever its lanes hold,
-//    so fragments loaded from memory for all 16 rows (zeros past M) cost
-//    the CU more load issue than its weights at small M.  Otherwise the
-//    fragments are read through a buffer resource of M * K fp16, so that
-//    rows past M read as zeros without a branch.
+//    registers for the whole kernel.  Every 16-byte load through the vector
+//    memory path costs that path 16 cycles whatever its lanes hold, so
+//    fragments loaded for all 16 rows (zeros past M) cost the CU more load
+//    issue than its weights at small M.  Hence three ways (SkinnyX):
+//    - M <= 8 (kXHalf): the lanes of rows 8..15 load rows 0..7 of the next
+//      fragment, so that one load fills two; a row rotation by 8 lanes (DPP)
+//      gives the second.  The tile's rows 8..15 then hold other rows' data,
+//      which reaches only outputs that are not stored.  Against X in LDS at
+//      M = 8: Llama down 10.2 -> 9.5 us, 16384 x 4096 16.9 -> 13.2, 12000 x
+//      6144 21.7 -> 17.7, the gate/up pairs and q|k|v within 2%; and half the
+//      X registers, so that 16 waves reach K = 14336 (4096 rows at M = 2 / 8:
+//      13.0 / 16.9 us against the GEMM's 32).
+//    - one tile of 9..16 rows that fit (kXLds): the block first copies the M
+//      real rows to LDS (rows padded by 16 bytes: the 16 rows of a fragment
+//      read hit distinct banks), before its weight loads, and each wave reads
+//      its fragments from there; rows past M read row 0.
+//    - otherwise (kXRegs) all 16 rows of a tile are read through a buffer
+//      resource of M * K fp16, so that rows past M read as zeros.
 //  * Each word is dequantized in registers without leaving fp16: its
 //    nibbles are spread to bytes (q0 q2 q4 q6 and q1 q3 q5 q7), and
 //    v_cvt_scalef32_pk_f16_fp8 turns two bytes into two fp16 at a time: read
@@ -68,11 +76,12 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
 // W waves, MT tiles of 16 activation rows, STEPS 128-wide k-steps per wave,
 // PAIR: two weight sets (gate, up) and a gated epilogue, RT tiles of 16
 // weight rows per block.  OCC: blocks per CU the register budget is sized for.
-template <int W, int MT, int STEPS, bool PAIR, int RT, int OCC, bool XL>
+template <int W, int MT, int STEPS, bool PAIR, int RT, int OCC, int XM>
 __global__ __launch_bounds__(64 * W, OCC) void q4_skinny_kernel(GemmParams p) {
     constexpr int NS = PAIR ? 2 : 1;
     constexpr int ROWS = 16 * RT;
-    static_assert(!XL || MT == 1, "LDS X holds one 16-row tile");
+    constexpr bool XL = XM == kXLds, XH = XM == kXHalf;
+    static_assert(XM == kXRegs || MT == 1, "one 16-row tile");
     __shared__ f32x4 red[W][RT][NS][MT][64];
     // [2 * NS slabs][ROWS][groups] fp16, then (XL) X rows [M][K + 8] fp16
     extern __shared__ u32x4 sb_lds[];
@@ -123,15 +132,27 @@ __global__ __launch_bounds__(64 * W, OCC) void q4_skinny_kernel(GemmParams p) {
     if constexpr (!XL) {
         const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<void*>(p.a), (short)0, p.M * K * 2, 0x00020000);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            const int xrow = ((mt * 16 + r16) * K + kw0) * 2;
+        if constexpr (XH) {
+            // lanes with r16 >= 8 take row r16 - 8 of the next fragment
+            const int xrow = ((r16 & 7) * K + kw0 + (r16 & 8)) * 2;
 #pragma unroll
             for (int t = 0; t < STEPS; ++t)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    xa[mt][t][r] = __builtin_bit_cast(
+                for (int r = 0; r < 4; r += 2)
+                    xa[0][t][r] = __builtin_bit_cast(
                         u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, xrow + 256 * t + 16 * r, 0, 0));
+        } else {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const int xrow = ((mt * 16 + r16) * K + kw0) * 2;
+#pragma unroll
+                for (int t = 0; t < STEPS; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        xa[mt][t][r] = __builtin_bit_cast(
+                            u32x4,
+                            __builtin_amdgcn_raw_buffer_load_b128(xrs, xrow + 256 * t + 16 * r, 0, 0));
+            }
         }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -178,22 +199,17 @@ __global__ __launch_bounds__(64 * W, OCC) void q4_skinny_kernel(GemmParams p) {
     // of the loads in flight and waits for all of them at the next use.  The
     // barrier is assembly with a memory clobber, so that no LDS read moves
     // above it.
-    __builtin_amdgcn_s_waitcnt(vmcnt_only((XL ? 0 : MT * STEPS * 4) + STEPS * RT * NS));
+    __builtin_amdgcn_s_waitcnt(vmcnt_only((XL ? 0 : XH ? STEPS * 2 : MT * STEPS * 4) + STEPS * RT * NS));
     __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 
-    if constexpr (XL) {   // rows past M read row 0 and are replaced by zeros
-        const bool live = r16 < p.M;
-        const u32x4* xr = xl + (live ? r16 : 0) * xrow16 + kw0 / 8;
-        const u32x4 zero = {0u, 0u, 0u, 0u};
+    if constexpr (XL) {   // rows past M (outputs that are not stored) read row 0
+        const u32x4* xr = xl + (r16 < p.M ? r16 : 0) * xrow16 + kw0 / 8;
 #pragma unroll
         for (int t = 0; t < STEPS; ++t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const u32x4 v = xr[16 * t + r];
-                xa[0][t][r] = live ? v : zero;
-            }
+            for (int r = 0; r < 4; ++r) xa[0][t][r] = xr[16 * t + r];
     }
 
 #pragma unroll
@@ -201,7 +217,16 @@ __global__ __launch_bounds__(64 * W, OCC) void q4_skinny_kernel(GemmParams p) {
 #pragma unroll
         for (int t = 0; t < STEPS; ++t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) xa[mt][t][r] = permute_x(xa[mt][t][r]);
+            for (int r = 0; r < 4; ++r) {
+                if (XH && (r & 1)) {   // rows 8.. of the fragment before (rows 8.. here unused)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        xa[mt][t][r][c] = (uint32_t)__builtin_amdgcn_mov_dpp((int)xa[mt][t][r - 1][c],
+                                                                            0x128, 0xF, 0xF, true);
+                } else {
+                    xa[mt][t][r] = permute_x(xa[mt][t][r]);
+                }
+            }
 
     const uint16_t* sbl = reinterpret_cast<const uint16_t*>(sb_lds);
     const int gshift = 5 + p.gshift;   // log2(group size)
@@ -292,12 +317,12 @@ __global__ __launch_bounds__(64 * W, OCC) void q4_skinny_kernel(GemmParams p) {
 
 // Registers of a configuration, roughly: X fragments, the packed words in
 // flight, accumulators, and about 40 for the rest.
-constexpr int skinny_vgprs(int mt, int steps, int ns, int rt) {
-    return 16 * mt * steps + 4 * rt * ns * steps + 4 * rt * ns * mt + 40;
+constexpr int skinny_vgprs(int mt, int steps, int ns, int rt, int xm = kXRegs) {
+    return (xm == kXHalf ? 8 : 16) * mt * steps + 4 * rt * ns * steps + 4 * rt * ns * mt + 40;
 }
 constexpr int kSkinnyMaxVgprs = 224;   // of the 256 one block of 8 waves may use
 
-// Dynamic LDS of a launch: the scale / bias slabs, then (XL) X's rows.
+// Dynamic LDS of a launch: the scale / bias slabs, then (kXLds) X's rows.
 size_t skinny_lds(const GemmParams& p, int rt, bool pair, bool xl) {
     return (size_t)(pair ? 4 : 2) * slab_alloc(16 * rt, p.groups) * 16 +
            (xl ? (size_t)p.M * (p.K / 8 + 1) * 16 : 0);
@@ -305,25 +330,32 @@ size_t skinny_lds(const GemmParams& p, int rt, bool pair, bool xl) {
 
 // Blocks per CU a configuration is compiled for: two when a wave fits in
 // 128 VGPRs.
-constexpr int skinny_occ(int w, int mt, int steps, int ns, int rt) {
-    return (w == 8 && skinny_vgprs(mt, steps, ns, rt) <= 120) ? 2 : 1;
+constexpr int skinny_occ(int w, int mt, int steps, int ns, int rt, int xm) {
+    return (w == 8 && skinny_vgprs(mt, steps, ns, rt, xm) <= 120) ? 2 : 1;
 }
 
-template <int W, int MT, int STEPS, bool PAIR, int RT, bool XL>
+template <int W, int MT, int STEPS, bool PAIR, int RT, int XM>
 hipError_t launch_cfg(const GemmParams& p, hipStream_t st) {
-    constexpr int OCC = skinny_occ(W, MT, STEPS, PAIR ? 2 : 1, RT);
+    constexpr int OCC = skinny_occ(W, MT, STEPS, PAIR ? 2 : 1, RT, XM);
     const dim3 grid((unsigned)((p.N + 16 * RT - 1) / (16 * RT))), block(64 * W);
-    const size_t lds = skinny_lds(p, RT, PAIR, XL);
-    hipLaunchKernelGGL((q4_skinny_kernel<W, MT, STEPS, PAIR, RT, OCC, XL>), grid, block, lds, st, p);
+    const size_t lds = skinny_lds(p, RT, PAIR, XM == kXLds);
+    hipLaunchKernelGGL((q4_skinny_kernel<W, MT, STEPS, PAIR, RT, OCC, XM>), grid, block, lds, st, p);
     return hipGetLastError();
 }
 
 template <int W, int MT, int STEPS, bool PAIR, int RT>
-hipError_t launch_xl(const GemmParams& p, bool xl, hipStream_t st) {
+hipError_t launch_x(const GemmParams& p, int xm, hipStream_t st) {
     if constexpr (MT == 1) {
-        if (xl) return launch_cfg<W, MT, STEPS, PAIR, RT, true>(p, st);
+        if (xm == kXHalf) return launch_cfg<W, MT, STEPS, PAIR, RT, kXHalf>(p, st);
     }
-    return launch_cfg<W, MT, STEPS, PAIR, RT, false>(p, st);
+    if constexpr (STEPS > (W == 8 ? 6 : 5)) {
+        return hipErrorInvalidValue;
+    } else {
+        if constexpr (MT == 1 && W == 8) {   // (16 waves: more than 8 rows of their K don't fit)
+            if (xm == kXLds) return launch_cfg<W, MT, STEPS, PAIR, RT, kXLds>(p, st);
+        }
+        return launch_cfg<W, MT, STEPS, PAIR, RT, kXRegs>(p, st);
+    }
 }
 
 template <int W, int MT, int STEPS>
@@ -331,16 +363,16 @@ hipError_t launch_steps(const GemmParams& p, const SkinnyPlan& pl, hipStream_t s
     const bool pair = p.w1 != nullptr;
     if (pl.RT == 2) {
         if constexpr (W == 8 && skinny_vgprs(MT, STEPS, 2, 2) <= kSkinnyMaxVgprs)
-            return pair ? launch_xl<W, MT, STEPS, true, 2>(p, pl.XL, st)
-                        : launch_xl<W, MT, STEPS, false, 2>(p, pl.XL, st);
+            return pair ? launch_x<W, MT, STEPS, true, 2>(p, pl.XM, st)
+                        : launch_x<W, MT, STEPS, false, 2>(p, pl.XM, st);
         return hipErrorInvalidValue;
     }
     if (pair) {
         // a gated pair of 5 steps does not fit the 128 VGPRs of 16 waves
-        if constexpr (W == 16 && STEPS == 5) return hipErrorInvalidValue;
-        else return launch_xl<W, MT, STEPS, true, 1>(p, pl.XL, st);
+        if constexpr (W == 16 && STEPS >= 5) return hipErrorInvalidValue;
+        else return launch_x<W, MT, STEPS, true, 1>(p, pl.XM, st);
     }
-    return launch_xl<W, MT, STEPS, false, 1>(p, pl.XL, st);
+    return launch_x<W, MT, STEPS, false, 1>(p, pl.XM, st);
 }
 
 }  // namespace
@@ -355,13 +387,13 @@ bool skinny_plan(const GemmParams& p, bool a_bf16, SkinnyPlan* out) {
         p.epilogue != kEpiResidual)
         return false;
     const int mt = p.M <= 16 ? 1 : 2;
-    SkinnyPlan pl{0, mt, 0, 1, 1, false};
+    SkinnyPlan pl{0, mt, 0, 1, 1, kXRegs};
     // 8 waves of 1..6 steps (1..4 with 32 activation rows), else 16 waves of
-    // 1..5 steps (1..4 for a gated pair; 16 activation rows)
+    // 4..5 steps (4 for a gated pair; one set of at most 8 rows 4..7)
     if (p.K % 1024 == 0 && p.K / 1024 <= (mt == 1 ? 6 : 4)) {
         pl.W = 8;
         pl.STEPS = p.K / 1024;
-    } else if (mt == 1 && p.K % 2048 == 0 && p.K / 2048 <= (pair ? 4 : 5)) {
+    } else if (mt == 1 && p.K % 2048 == 0 && p.K / 2048 <= (pair ? 4 : p.M <= 8 ? 7 : 5)) {
         // (a gated pair of 5 steps does not fit the 128 VGPRs of 16 waves)
         pl.W = 16;
         pl.STEPS = p.K / 2048;
@@ -371,20 +403,27 @@ bool skinny_plan(const GemmParams& p, bool a_bf16, SkinnyPlan* out) {
     // Two row tiles per block (the X slice serves twice the weight rows), with
     // 8 waves and at least one block per CU: when the two-tile block still
     // fits two per CU, or above 8 activation rows.  Measured: the vocabulary
-    // head at M = 2 takes 43.8 us with two tiles (two blocks per CU) against
-    // 53.5 us with one; the gate/up pair at M = 8 (two tiles: one block per
-    // CU) 10.6 against 10.1 us, at M = 16 11.2 against 12.4 us.
+    // head at M = 8 takes 59.3 us with two tiles (two blocks per CU) against
+    // 75.2 us with one, 16384 x 4096 13.2 against 15.0; the gate/up pair at
+    // M = 16 11.2 against 12.4.  A pair of at most 8 rows keeps one tile:
+    // 10.8 against 11.3 us (8192 x 3072), 6.3 against 6.9 (12000 x 1024).
     const int ns = pair ? 2 : 1;
+    pl.XM = p.M <= 8 ? kXHalf : kXRegs;
     // (launch_steps instantiates two tiles where a gated pair of them fits
     // the register budget; every two-tile block that fits two per CU does)
-    if (pl.W == 8 && (p.N + 31) / 32 >= kCUs &&
-        (skinny_occ(8, mt, pl.STEPS, ns, 2) == 2 ||
+    if (pl.W == 8 && !(pair && pl.XM == kXHalf) && (p.N + 31) / 32 >= kCUs &&
+        (skinny_occ(8, mt, pl.STEPS, ns, 2, pl.XM) == 2 ||
          (p.M > 8 && skinny_vgprs(mt, pl.STEPS, 2, 2) <= kSkinnyMaxVgprs)))
         pl.RT = 2;
-    pl.OCC = skinny_occ(pl.W, mt, pl.STEPS, ns, pl.RT);
-    // X in LDS: one 16-row tile whose rows fit beside the slabs, so that a
-    // block still gets its share of the CU's LDS
-    pl.XL = mt == 1 && skinny_lds(p, pl.RT, pair, true) <= (size_t)(pl.RT == 2 ? 128 : 64) * 1024;
+    pl.OCC = skinny_occ(pl.W, mt, pl.STEPS, ns, pl.RT, pl.XM);
+    // X of 9..16 rows in LDS: where the rows fit beside the slabs, so that a
+    // block still gets its share of the CU's LDS (all of it where the grid has
+    // no second block for a CU: 3072 x 3072 at M = 16 takes 5.6 us with X in
+    // LDS, 6.2 without).
+    if (pl.W == 8 && mt == 1 && pl.XM == kXRegs &&
+        skinny_lds(p, pl.RT, pair, true) <=
+            (size_t)(pl.RT == 2 || (p.N + 15) / 16 <= kCUs ? 128 : 64) * 1024)
+        pl.XM = kXLds;
     // scales and biases are staged with 16-byte loads
     const uintptr_t sb = reinterpret_cast<uintptr_t>(p.s0) | reinterpret_cast<uintptr_t>(p.b0) |
                          (pair ? reinterpret_cast<uintptr_t>(p.s1) | reinterpret_cast<uintptr_t>(p.b1)
@@ -413,11 +452,10 @@ hipError_t launch_skinny(const GemmParams& p, const SkinnyPlan& pl, hipStream_t 
         }
     } else if (pl.W == 16 && pl.MT == 1) {
         switch (pl.STEPS) {
-            case 1: return launch_steps<16, 1, 1>(p, pl, st);
-            case 2: return launch_steps<16, 1, 2>(p, pl, st);
-            case 3: return launch_steps<16, 1, 3>(p, pl, st);
             case 4: return launch_steps<16, 1, 4>(p, pl, st);
             case 5: return launch_steps<16, 1, 5>(p, pl, st);
+            case 6: return launch_steps<16, 1, 6>(p, pl, st);
+            case 7: return launch_steps<16, 1, 7>(p, pl, st);
         }
     }
     return hipErrorInvalidValue;
