@@ -900,7 +900,13 @@ int sltx_matmul_q4_residual_rms_norm(const void* x, const sltx_q4_weight* w, con
     // Llama o 7.4 / 8.7 / 10.2 / 15.6 / 19.7 / 22.1 against 17.2 / 17.9 / 18.6 /
     // 19.6 / 23.6 / 27.0 at M = 2 / 8 / 32 / 64 / 128 / 256; Llama down 10.4 /
     // 13.7 / 15.8 / 19.5 / 24.8 / 33.0 against 23.2 / 23.6 / 24.7 / 26.2 / 29.8 /
-    // 33.7.  (Under capture without a workspace the call has already failed,
+    // 33.7.  An unsplit GEMM and the norm against split partials and the fused pass:
+    // 2048 x 2048 at M = 500 / 1200 15.9 / 26.1 against 24.1 / 29.4, 4096 x 3072 at
+    // M = 700 / 1100 34.0 / 47.5 against 35.9 / 49.3; the slower one only around
+    // 4096 x 4096 at M = 700..1024 (44.8 - 53.3 against 43.8 - 52.4), where the
+    // unfused product is the faster unsplit (47 against 50) and both calls plan
+    // alike so that their results agree bit for bit.
+    // (Under capture without a workspace the call has already failed,
     // as it does for every shape.)
     NarrowPlan np;
     SkinnyPlan sp;
