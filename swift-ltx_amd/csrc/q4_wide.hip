@@ -160,7 +160,7 @@ __global__ __launch_bounds__(WT, 1) void q4_wide_kernel(GemmParams p, WideArgs w
     __shared__ u32x4 xs0[XS], xs1[XS], xs2[XS], xs3[NSX > 3 ? XS : 1];
     __shared__ uint32_t ws0[WDW], ws1[WDW], ws2[WDW], ws3[NSX > 3 ? WDW : 1];
     __shared__ __align__(16) uint32_t slab[SLAB_G * WBN];
-    
+
     auto xstage = [&](auto sc) -> u32x4* {
         constexpr int S = decltype(sc)::value % NSX;
         if constexpr (S == 0) return xs0;
@@ -547,7 +547,7 @@ bool wide_plan(const GemmParams& p, bool a_bf16, WidePlan* out) {
     // K of one block: a slab of at most SLAB_G groups, and no more than
     // measured (4096; group 128 at M <= 256: 8192)
     const int kmax = p.M <= 256 && g == 128 ? 8192 : 4096;
-    
+
     const long nblocks = ((long)p.N + (pair ? 31 : WBN - 1)) / (pair ? 32 : WBN);
     const long most = p.M <= 64 ? 2 * kCUs : kCUs;
     double best_us = 1e30;
