@@ -8,7 +8,9 @@ csrc/bench/*.hip -> lib/libswiftltx_bench.so, measurement kernels that only
 bench.py loads (the HBM read ceiling); not part of the C ABI.
 csrc/py/q4_binding.cpp -> lib/_q4_binding.so, the native marshalling of the
 Python mirror's hot calls (a CPython extension over torch's C++ tensors; host
-code, built with g++ where torch is installed).
+code, built with g++ where torch is installed).  The mirror works without it
+(through ctypes), so where it cannot be built the libraries still are, with a
+warning.
 Objects go to swift-ltx_amd/_build/, the libraries to swift-ltx_amd/lib/.
 Every HIP file is compiled for gfx950 only, with packed-fp32 instruction
 selection disabled (hipcc's host pass warns that it does not know the
@@ -20,6 +22,7 @@ import concurrent.futures as cf
 import glob
 import importlib.util
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -58,13 +61,19 @@ def headers() -> list[str]:
             + sorted(glob.glob(os.path.join(REPO, "include", "*.h"))))
 
 
-def is_stale() -> bool:
-    outputs = [LIB_PATH, BENCH_LIB_PATH] + ([BINDING_PATH] if torch_dir() else [])
+def _older(outputs: list[str], inputs: list[str]) -> bool:
     if not all(os.path.exists(f) for f in outputs):
         return True
     t = min(os.path.getmtime(f) for f in outputs)
-    return any(os.path.getmtime(f) > t
-               for f in sources() + bench_sources() + headers() + [BINDING_SRC, __file__])
+    return any(os.path.getmtime(f) > t for f in inputs)
+
+
+def libs_stale() -> bool:
+    return _older([LIB_PATH, BENCH_LIB_PATH], sources() + bench_sources() + headers() + [__file__])
+
+
+def binding_stale() -> bool:
+    return torch_dir() is not None and _older([BINDING_PATH], headers() + [BINDING_SRC, __file__])
 
 
 def torch_dir() -> str | None:
@@ -81,7 +90,8 @@ def _build_binding() -> None:
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
            "-I" + os.path.join(REPO, "include"), "-I" + os.path.join(t, "include"),
            "-I" + os.path.join(t, "include", "torch", "csrc", "api", "include"),
-           "-I" + sysconfig.get_paths()["include"], "-isystem", "/opt/rocm/include",
+           "-I" + sysconfig.get_paths()["include"],
+           "-isystem", os.path.join(os.path.dirname(os.path.dirname(shutil.which(HIPCC) or HIPCC)), "include"),
            BINDING_SRC, "-o", tmp, "-L" + os.path.join(t, "lib"),
            "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -115,18 +125,29 @@ def _link(objs: list[str], path: str) -> None:
 
 def build(force: bool = True, jobs: int = 8) -> str:
     """Compile every csrc/*.hip (and csrc/bench/*.hip) for gfx950, link
-    LIB_PATH and BENCH_LIB_PATH, and build BINDING_PATH; returns LIB_PATH."""
-    if not force and not is_stale():
+    LIB_PATH and BENCH_LIB_PATH, and build BINDING_PATH where that can be done;
+    returns LIB_PATH."""
+    libs, binding = force or libs_stale(), force or binding_stale()
+    if not libs and not binding:
         return LIB_PATH
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
-    main, bench = sources(), bench_sources()
     with cf.ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
-        binding = ex.submit(_build_binding)
-        objs = list(ex.map(_compile, main + bench))
-        binding.result()
-    _link(objs[:len(main)], LIB_PATH)
-    _link(objs[len(main):], BENCH_LIB_PATH)
+        built = ex.submit(_build_binding) if binding else None
+        if libs:
+            main, bench = sources(), bench_sources()
+            objs = list(ex.map(_compile, main + bench))
+            _link(objs[:len(main)], LIB_PATH)
+            _link(objs[len(main):], BENCH_LIB_PATH)
+    try:
+        if built is not None:
+            built.result()
+    except (RuntimeError, OSError) as e:
+        # no g++, Python headers or ROCm torch, say.  One built from other
+        # sources may not fit the library: it goes.
+        if os.path.exists(BINDING_PATH):
+            os.remove(BINDING_PATH)
+        sys.stderr.write(f"warning: {BINDING_PATH} not built, ctypes serves every call: {e}\n")
     return LIB_PATH
 
 
