@@ -3,7 +3,7 @@ Ops entry points over the C ABI in include/swiftltx_q4.h.
 
 The shipped compute path is libswiftltx_q4.so (hand-written HIP for gfx950);
 this module only marshals torch device tensors into it: plain calls through
-lib/_q4_binding.so (csrc/py/q4_binding.cpp), everything else, and every error,
+lib/_q4_binding.*.so (csrc/py/q4_binding.cpp), everything else, and every error,
 through ctypes.  There is no fallback for the library: if it is missing, every
 entry point raises.
 
@@ -196,28 +196,41 @@ def lib():
 # counterpart's result, or None for anything but the plain accepted call, which
 # then goes on in Python.  A matmul_q4 call took 12 us of host time through
 # ctypes (kernel: 3.3 us), a layer of five calls 73 us.
-BINDING_PATH = os.path.join(PKG_DIR, "lib", "_q4_binding.so")
 _native = None
 _native_tried = False
+
+
+def _binding_path():
+    """The binding built for this Python and this torch (build.py names it after
+    both): another one's inlined reads of a tensor may not fit."""
+    import sysconfig
+    v = _torch().version
+    return os.path.join(PKG_DIR, "lib", "_q4_binding.%s.torch-%s-%s.so" % (
+        sysconfig.get_config_var("SOABI"), v.__version__, (getattr(v, "git_version", None) or "")[:8]))
 
 
 def _load_binding():
     global _native, _native_tried
     _native_tried = True
-    if not os.path.exists(BINDING_PATH):
-        return
+    import glob
     import importlib.util
     import warnings
-    _torch()   # the binding links against its libraries (and the library takes its HIP runtime)
+    path = _binding_path()   # (imports torch, whose HIP runtime the library takes)
+    if not os.path.exists(path):
+        others = glob.glob(os.path.join(os.path.dirname(path), "_q4_binding*.so"))
+        if others:
+            warnings.warn(f"{', '.join(others)} not loaded: built against another Python or torch "
+                          "(ctypes serves every call)")
+        return
     L = lib()
     try:
-        spec = importlib.util.spec_from_file_location("_q4_binding", BINDING_PATH)
+        spec = importlib.util.spec_from_file_location("_q4_binding", path)
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
         mod.init({n: ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in EXPORTED
                   if not n.startswith("sltx_st_")}, check, Q4Weight)
-    except (ImportError, KeyError) as e:   # built against another torch: ctypes serves every call
-        warnings.warn(f"{BINDING_PATH} not loaded: {e}")
+    except (ImportError, KeyError) as e:
+        warnings.warn(f"{path} not loaded: {e}")
         return
     _native = mod
 

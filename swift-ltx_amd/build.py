@@ -6,11 +6,13 @@
 csrc/*.hip -> lib/libswiftltx_q4.so, the drop-in library (include/swiftltx_q4.h).
 csrc/bench/*.hip -> lib/libswiftltx_bench.so, measurement kernels that only
 bench.py loads (the HBM read ceiling); not part of the C ABI.
-csrc/py/q4_binding.cpp -> lib/_q4_binding.so, the native marshalling of the
-Python mirror's hot calls (a CPython extension over torch's C++ tensors; host
-code, built with g++ where torch is installed).  The mirror works without it
-(through ctypes), so where it cannot be built the libraries still are, with a
-warning.
+csrc/py/q4_binding.cpp -> lib/_q4_binding.<Python ABI>.torch-<version>.so, the
+native marshalling of the Python mirror's hot calls (a CPython extension over
+torch's C++ tensors; host code, built with g++ where torch is installed).  It
+reads tensors through torch's inlined accessors, so it serves only the Python
+and the torch that it was built against: its name holds both, and the mirror
+looks for the name of its own.  The mirror works without it (through ctypes),
+so where it cannot be built the libraries still are, with a warning.
 Objects go to swift-ltx_amd/_build/, the libraries to swift-ltx_amd/lib/.
 Every HIP file is compiled for gfx950 only, with packed-fp32 instruction
 selection disabled (hipcc's host pass warns that it does not know the
@@ -22,6 +24,7 @@ import concurrent.futures as cf
 import glob
 import importlib.util
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -35,7 +38,6 @@ LIB_DIR = os.path.join(PKG, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libswiftltx_q4.so")
 BENCH_LIB_PATH = os.path.join(LIB_DIR, "libswiftltx_bench.so")
 BINDING_SRC = os.path.join(CSRC, "py", "q4_binding.cpp")
-BINDING_PATH = os.path.join(LIB_DIR, "_q4_binding.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 DEVICE_FLAGS = [
@@ -73,7 +75,8 @@ def libs_stale() -> bool:
 
 
 def binding_stale() -> bool:
-    return torch_dir() is not None and _older([BINDING_PATH], headers() + [BINDING_SRC, __file__])
+    path = binding_path()
+    return path is not None and _older([path], headers() + [BINDING_SRC, __file__])
 
 
 def torch_dir() -> str | None:
@@ -82,11 +85,25 @@ def torch_dir() -> str | None:
     return os.path.dirname(spec.origin) if spec and spec.origin else None
 
 
-def _build_binding() -> None:
+def binding_path() -> str | None:
+    """The binding's path for this Python and the installed torch (None without
+    one): the name __init__.py looks for.  Of torch, the version and the commit,
+    read from its version.py."""
     t = torch_dir()
-    if not t:
-        return
-    tmp = BINDING_PATH + ".tmp%d" % os.getpid()
+    if not t or not os.path.exists(os.path.join(t, "version.py")):
+        return None
+    text = open(os.path.join(t, "version.py")).read()
+    version, commit = (re.search(rf"^{k}\b[^=\n]*=\s*'([^']*)'", text, re.M)
+                       for k in ("__version__", "git_version"))
+    if not version:
+        return None
+    return os.path.join(LIB_DIR, "_q4_binding.%s.torch-%s-%s.so" % (
+        sysconfig.get_config_var("SOABI"), version[1], commit[1][:8] if commit else ""))
+
+
+def _build_binding(path: str) -> None:
+    t = torch_dir()
+    tmp = path + ".tmp%d" % os.getpid()
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
            "-I" + os.path.join(REPO, "include"), "-I" + os.path.join(t, "include"),
            "-I" + os.path.join(t, "include", "torch", "csrc", "api", "include"),
@@ -97,7 +114,7 @@ def _build_binding() -> None:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"g++ failed for {BINDING_SRC}:\n{r.stderr}")
-    os.replace(tmp, BINDING_PATH)
+    os.replace(tmp, path)
 
 
 def _compile(src: str) -> str:
@@ -125,15 +142,16 @@ def _link(objs: list[str], path: str) -> None:
 
 def build(force: bool = True, jobs: int = 8) -> str:
     """Compile every csrc/*.hip (and csrc/bench/*.hip) for gfx950, link
-    LIB_PATH and BENCH_LIB_PATH, and build BINDING_PATH where that can be done;
+    LIB_PATH and BENCH_LIB_PATH, and build the binding where that can be done;
     returns LIB_PATH."""
-    libs, binding = force or libs_stale(), force or binding_stale()
+    path = binding_path()
+    libs, binding = force or libs_stale(), path is not None and (force or binding_stale())
     if not libs and not binding:
         return LIB_PATH
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     with cf.ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
-        built = ex.submit(_build_binding) if binding else None
+        built = ex.submit(_build_binding, path) if binding else None
         if libs:
             main, bench = sources(), bench_sources()
             objs = list(ex.map(_compile, main + bench))
@@ -143,11 +161,14 @@ def build(force: bool = True, jobs: int = 8) -> str:
         if built is not None:
             built.result()
     except (RuntimeError, OSError) as e:
-        # no g++, Python headers or ROCm torch, say.  One built from other
-        # sources may not fit the library: it goes.
-        if os.path.exists(BINDING_PATH):
-            os.remove(BINDING_PATH)
-        sys.stderr.write(f"warning: {BINDING_PATH} not built, ctypes serves every call: {e}\n")
+        # no g++, Python headers or ROCm torch, say
+        built = None
+        sys.stderr.write(f"warning: {path} not built, ctypes serves every call: {e}\n")
+    # Bindings of other builds, and one that could not be built again, may not
+    # fit the library.
+    for old in glob.glob(os.path.join(LIB_DIR, "_q4_binding*.so")):
+        if old != path or (binding and built is None):
+            os.remove(old)
     return LIB_PATH
 
 

@@ -11,8 +11,19 @@ from helpers import gpu_inputs
 def native(pkg):
     if not pkg._native_tried:
         pkg._load_binding()
-    assert pkg._native is not None, "lib/_q4_binding.so is not built"
+    assert pkg._native is not None, "lib/_q4_binding.*.so is not built"
     return pkg._native
+
+
+@pytest.mark.parametrize("attr,value", [("__version__", "9.9.0"), ("git_version", "0" * 40)])
+def test_another_torchs_binding_is_not_loaded(pkg, native, monkeypatch, attr, value):
+    """Its inlined reads of a tensor may not fit: ctypes serves the calls."""
+    import torch
+    monkeypatch.setattr(torch.version, attr, value)
+    monkeypatch.setattr(pkg, "_native", None)
+    with pytest.warns(UserWarning, match="another Python or torch"):
+        pkg._load_binding()
+    assert pkg._native is None
 
 
 def test_declines_host_tensors_and_other_types(pkg, native):
