@@ -118,8 +118,18 @@ int32_t dtype_code(at::ScalarType d) {
     return d == at::kHalf ? SLTX_F16 : d == at::kBFloat16 ? SLTX_BF16 : SLTX_F32;
 }
 
+// Without the interpreter lock while it lives.
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    Unlocked() = default;
+    Unlocked(const Unlocked&) = delete;
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 // The output the caller gave, or a new one: the object to return (owned) and
-// the address.
+// the address.  torch's allocator may wait for the GPU (to give cached blocks
+// back before it asks for more), so it runs without the interpreter lock, as
+// torch.empty runs it.
 struct Out {
     PyObject* obj = nullptr;
     void* ptr = nullptr;
@@ -136,7 +146,11 @@ struct Out {
         for (int64_t s : shape) n *= s;
         if (o == Py_None) {
             need(like.is_cuda());
-            at::Tensor t = at::empty(shape, at::TensorOptions().dtype(d).device(like.device()));
+            at::Tensor t;
+            {
+                Unlocked unlocked;
+                t = at::empty(shape, at::TensorOptions().dtype(d).device(like.device()));
+            }
             ptr = t.data_ptr();
             obj = THPVariable_Wrap(std::move(t));
             if (!obj) throw Decline{};

@@ -120,3 +120,50 @@ def test_streams_outputs_and_errors(pkg, dev, native):
     with pytest.raises(pkg.SltxError) as e:
         pkg.matmul_q4(x, w, s, b, M, K, N, g, out=x.view(-1)[: M * N].view(M, N))
     assert e.value.code == pkg.SLTX_ERR_INVALID and "overlaps" in str(e.value)
+
+
+@pytest.mark.gpu
+def test_other_threads_run_while_an_output_is_allocated(pkg, dev, native):
+    """Within a limit that holds either a cached block or the new output, the
+    allocator gives the block back, which waits for the GPU's queued work: about a
+    second here.  Another Python thread goes on meanwhile."""
+    import threading
+    import time
+    import torch
+    a = torch.zeros(48 << 20, device=dev, dtype=torch.float16)
+    m = torch.zeros(8192, 8192, device=dev, dtype=torch.float16)
+    r = torch.empty_like(m)
+    torch.mm(m, m, out=r)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    cached = torch.empty(64 << 20, device=dev, dtype=torch.uint8)
+    del cached   # 64 MB kept by the allocator; the output takes 96 MB
+    total = torch.cuda.get_device_properties(dev).total_memory
+    gap, stop = [0.0], threading.Event()
+
+    def tick():
+        last = time.perf_counter()
+        while not stop.is_set():
+            time.sleep(0.001)
+            now = time.perf_counter()
+            gap[0] = max(gap[0], now - last)
+            last = now
+
+    t = threading.Thread(target=tick)
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (48 << 20)) / total)
+    try:
+        for _ in range(800):
+            torch.mm(m, m, out=r)
+        t.start()
+        begin = time.perf_counter()
+        out = pkg.silu_mul(a, a)
+        took = time.perf_counter() - begin
+    finally:
+        stop.set()
+        if t.ident is not None:
+            t.join()
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        torch.cuda.synchronize()
+    assert not out.any()
+    assert took > 0.2, f"the allocator did not wait ({took:.3f} s)"
+    assert gap[0] < took / 2, f"another thread stood still for {gap[0]:.3f} of {took:.3f} s"
