@@ -373,7 +373,7 @@ int run_gemm(const char* fn, const void* x, int x_dtype, const sltx_q4_weight& w
         }
         return finish(launch_wide(p, wp, st), fn);
     }
-    if (strip_ok(p)) return finish(launch_strip(p, st), fn);
+    if (strip_rows(p)) return finish(launch_strip(p, st), fn);
     const size_t need = gemm_workspace_bytes(p);
     if (need > 0) p.ws = stream_workspace(st, need);
     return finish(launch_gemm(p, x_dtype == kBF16, st), fn);
@@ -932,19 +932,18 @@ int sltx_matmul_q4_residual_rms_norm(const void* x, const sltx_q4_weight* w, con
                   fn);
 }
 
-int sltx_gemm_route(int32_t M, int32_t N, int32_t K, int32_t group_size, int32_t gated,
-                    int32_t x_dtype) {
-    const char* fn = "sltx_gemm_route";
+// Operands of sltx_gemm_route's shape at 256-byte aligned stand-in addresses (the
+// plans read only the shape and the pointers' alignment); kOk, or the error.
+static int shape_params(const char* fn, int M, int N, int K, int group_size, bool gated, int x_dtype,
+                        GemmParams& p) {
     if (M < 1 || N < 1 || K <= 0 || K % 32 != 0)
         return fail(kErrInvalid, "%s: M, N must be >= 1 and K a positive multiple of 32", fn);
     if (group_size <= 0 || K % group_size != 0 || log2_group(group_size) < 0)
         return fail(kErrInvalid, "%s: group_size must be 32, 64 or 128 and divide K", fn);
     if (x_dtype != kF16 && x_dtype != kBF16 && x_dtype != kF32)
         return fail(kErrInvalid, "%s: bad x_dtype", fn);
-    // operands at 256-byte aligned stand-in addresses: the plans read only
-    // the shape and the pointers' alignment
     const void* al = reinterpret_cast<const void*>(uintptr_t{256});
-    GemmParams p{};
+    p = GemmParams{};
     p.a = al;
     p.w0 = static_cast<const uint32_t*>(al);
     p.s0 = p.b0 = static_cast<const uint16_t*>(al);
@@ -960,10 +959,49 @@ int sltx_gemm_route(int32_t M, int32_t N, int32_t K, int32_t group_size, int32_t
     p.splits = 1;
     // fp32 x: wide outputs are cast once and take the fp16 routes
     p.a_f32 = x_dtype == kF32 && N <= 2 * 256 ? 1 : 0;
+    return kOk;
+}
+
+int sltx_gemm_route(int32_t M, int32_t N, int32_t K, int32_t group_size, int32_t gated,
+                    int32_t x_dtype) {
+    GemmParams p;
+    const int rc = shape_params("sltx_gemm_route", M, N, K, group_size, gated != 0, x_dtype, p);
+    if (rc != kOk) return rc;
     NarrowPlan np;
     SkinnyPlan sp;
     WidePlan wp;
     return gemm_route(p, x_dtype == kBF16, &np, &sp, &wp);
+}
+
+// For the tests, and so not in the public header: what run_gemm plans, as
+// {sltx_gemm_route, K splits across blocks, and, of the wide route, the GEMM and
+// its strip kernel (the one with fewer than 128 rows), the activation and the
+// weight rows of a block, else 0}.
+int sltx_internal_plan(int32_t M, int32_t N, int32_t K, int32_t group_size, int32_t gated, int32_t x_dtype,
+                       int32_t out[4]) {
+    GemmParams p;
+    const int rc = shape_params("sltx_internal_plan", M, N, K, group_size, gated != 0, x_dtype, p);
+    if (rc != kOk) return rc;
+    NarrowPlan np;
+    SkinnyPlan sp;
+    WidePlan wp;
+    out[0] = gemm_route(p, x_dtype == kBF16, &np, &sp, &wp);
+    out[1] = 1;
+    out[2] = out[3] = 0;
+    if (out[0] == SLTX_ROUTE_MID) {
+        out[1] = mid_splits(p);
+    } else if (out[0] == SLTX_ROUTE_WIDE) {
+        out[1] = wp.splits;
+        out[2] = 32 * wp.tm;
+        out[3] = 64;
+    } else if (out[0] == SLTX_ROUTE_GEMM && strip_rows(p)) {
+        out[2] = strip_rows(p);
+        out[3] = 128;
+    } else if (out[0] == SLTX_ROUTE_GEMM) {
+        out[1] = gemm_splits(p);
+        gemm_tile(p, &out[2], &out[3]);
+    }
+    return kOk;
 }
 
 }  // extern "C"

@@ -258,6 +258,11 @@ static GemmPlan plan_gemm(const GemmParams& p, bool allow_split) {
 
 size_t gemm_workspace_bytes(const GemmParams& p) { return plan_gemm(p, true).ws_bytes; }
 int gemm_splits(const GemmParams& p) { return plan_gemm(p, true).splits; }
+void gemm_tile(const GemmParams& p, int* rows, int* wrows) {
+    const GemmPlan pl = plan_gemm(p, true);
+    *rows = 64 * pl.wm;
+    *wrows = BN / pl.kg;
+}
 size_t gemm_partials_workspace_bytes(const GemmParams& p) {
     return (size_t)gemm_splits(p) * p.M * p.N * sizeof(float);
 }

@@ -226,8 +226,8 @@ hipError_t launch_wide(GemmParams p, const WidePlan& pl, hipStream_t st);
 hipError_t launch_splitk_reduce(const GemmParams& p, hipStream_t st);
 
 // fp32 x and few output columns (q4_strip.hip): the GEMM family's kernel where
-// strip_ok.
-bool strip_ok(const GemmParams& p);
+// strip_rows, the activation rows of its blocks, is not 0.
+int strip_rows(const GemmParams& p);
 hipError_t launch_strip(GemmParams p, hipStream_t st);
 
 // Bytes of split-K workspace the launch of `p` would use (0: it does not split).
@@ -238,6 +238,8 @@ hipError_t launch_gemm(GemmParams p, bool a_bf16, hipStream_t st);
 // K splits of the GEMM's plan for p, and the bytes of fp32 partials they take
 // (counted for one split too).
 int gemm_splits(const GemmParams& p);
+// The activation and weight rows of that plan's tiles.
+void gemm_tile(const GemmParams& p, int* rows, int* wrows);
 size_t gemm_partials_workspace_bytes(const GemmParams& p);
 // GEMM of more than one K split (no epilogue; p.residual is the residual input) into the workspace
 // p.ws, then one pass per row: res_out = half(residual + half(sum of splits))

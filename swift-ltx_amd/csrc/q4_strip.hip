@@ -289,11 +289,11 @@ static int strip_height(const GemmParams& p) {
 // longer K wants more rows, since the GEMM splits K and this kernel does not:
 // at K = 4096, N = 128, M = 300 / 2000 / 6144 23.0 / 23.4 / 26.9 against 18.8 /
 // 23.0 / 38.4; N = 512, M = 300 / 1000 23.4 / 23.5 against 22.6 / 29.4.
-bool strip_ok(const GemmParams& p) {
-    if (!p.a_f32 || p.w1 != nullptr || (p.epilogue != kEpiNone && p.epilogue != kEpiGeluTanh)) return false;
-    if (p.M < 1 || p.N < 1 || p.N > 4 * SBN || p.K % RK != 0 || p.groups > SLAB_G) return false;
-    if (p.K > 4096 || (p.K > 2048 && (long)p.M * p.N < 1L << 18)) return false;
-    return strip_height(p) > 0 && (reinterpret_cast<uintptr_t>(p.a) & 15) == 0;
+int strip_rows(const GemmParams& p) {
+    if (!p.a_f32 || p.w1 != nullptr || (p.epilogue != kEpiNone && p.epilogue != kEpiGeluTanh)) return 0;
+    if (p.M < 1 || p.N < 1 || p.N > 4 * SBN || p.K % RK != 0 || p.groups > SLAB_G) return 0;
+    if (p.K > 4096 || (p.K > 2048 && (long)p.M * p.N < 1L << 18)) return 0;
+    return (reinterpret_cast<uintptr_t>(p.a) & 15) == 0 ? 32 * strip_height(p) : 0;
 }
 
 hipError_t launch_strip(GemmParams p, hipStream_t st) {

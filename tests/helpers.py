@@ -13,7 +13,9 @@ Tolerances (fp64 oracle = reference semantics w = s*q + b, exact):
 """
 from __future__ import annotations
 
+import ctypes
 import os
+from typing import NamedTuple
 
 import numpy as np
 from safetensors.numpy import load_file
@@ -98,3 +100,21 @@ def host(t):
     if t.dtype == torch.bfloat16:
         return t.view(torch.int16).cpu().numpy().view(np.uint16)
     return t.cpu().numpy()
+
+
+class Plan(NamedTuple):
+    """The kernel family, its K splits across blocks, and (wide route, GEMM and
+    strip kernel) the activation and weight rows of a block.  The strip kernel's
+    family is "gemm"; its 32 or 64 rows tell it from the GEMM's 128 or 192."""
+    route: str
+    splits: int
+    rows: int
+    wrows: int
+
+
+def plan(pkg, M, N, K, g=64, gated=False, x_dtype=None):
+    """What the library plans for a matmul of this shape (no device needed)."""
+    out = (ctypes.c_int32 * 4)()
+    code = pkg.SLTX_F16 if x_dtype is None else pkg._dtype_code(x_dtype)
+    pkg.check(pkg.lib().sltx_internal_plan(M, N, K, g, 1 if gated else 0, code, out))
+    return Plan(pkg.ROUTES[out[0]], *out[1:])

@@ -6,8 +6,8 @@ applies the epilogue; it also resets the counter for the next launch.
 
 Same semantics as every M > 1 route (matmulQ4Fast / matmulQ4FastF32,
 Ops.swift:312-381; the SwiGLU / GeGLU pairs, LlamaModel.swift:275-277,
-T5Encoder.swift:191-199).  Covered: 2, 3, 4 and 8 splits, one and two blocks
-along M, gated pairs, ragged and odd column counts (element loads and
+T5Encoder.swift:191-199).  Covered: 2, 3, 4 and 8 splits at each block
+height they are planned with, one to five blocks along M, gated pairs, ragged and odd column counts (element loads and
 stores), fp16 and fp32 outputs (which must agree bit for bit), launches
 back to back on one stream with different tile counts (the counters must
 return to zero after each), and split launches inside a HIP graph replayed
@@ -17,46 +17,48 @@ every repeat must equal the first result bit for bit.
 import numpy as np
 import pytest
 
-from helpers import GATE, TOL_GEMM_F16, assert_parity, to_dev
+from helpers import GATE, TOL_GEMM_F16, assert_parity, plan, to_dev
 from oracle import q4_oracle as o
 
 pytestmark = pytest.mark.gpu
 
 
-def wide_splits(M, N, K, g, pair):
-    """The K splits the wide route plans for this shape (its rule: split
-    while the blocks would not fill the GPU or a split's K range holds more
-    than 64 scale groups, in whole rounds of 128 k, up to 8 splits; three
-    instead of two where two leave a quarter of the CUs idle and three fit)."""
-    mblocks = -(-M // 128)
-    nblocks = -(-N // (32 if pair else 64))
-    if mblocks == 2 and 160 <= nblocks * 2 and nblocks * 3 <= 256:   # three M-blocks
-        mblocks = 3
-    blocks, rounds, s = nblocks * mblocks, K // 128, 1
-    while s < 8 and rounds % (2 * s) == 0 and (K // s // g > 64 or
-                                                (blocks * s < 160 and rounds // (2 * s) >= 4)):
-        s *= 2
-    if (s < 3 and blocks * s < 192 and blocks * 3 <= 256 and rounds % 3 == 0 and rounds // 3 >= 4
-            and K // 3 // g <= 64):
-        s = 3
-    return s
-
-
-# (M, N, K, g, epilogue, splits)
+# (M, N, K, g, epilogue, splits, activation rows of a block), as the library
+# plans them: every pair of split count and block height that it plans for one
+# set and for a gated pair
 CASES = [
-    (128, 5120, 3072, 64, None, 3),      # Llama q|k|v at M = 128
-    (64, 5101, 3072, 32, None, 3),       # three splits, odd N
-    (200, 2600, 3072, 64, None, 3),      # three splits, two blocks along M, ragged N
-    (128, 3072, 3072, 64, None, 4),      # Llama o
-    (128, 4096, 10240, 64, None, 4),     # T5 wo at M = 128
-    (64, 1024, 8192, 64, None, 8),
-    (200, 3072, 8192, 64, None, 2),      # two blocks along M
-    (100, 1000, 4096, 32, None, 8),      # ragged last column block
-    (64, 1001, 2048, 64, None, 4),       # odd N: element loads and stores
-    (128, 2560, 3072, 64, "gelu", 3),    # gated pairs
-    (96, 1024, 4096, 64, "silu", 8),
+    (128, 3072, 3072, 64, None, 2, 64),      # Llama o
+    (64, 1001, 2048, 64, None, 2, 64),       # odd N: element loads and stores
+    (64, 5101, 3072, 32, None, 3, 64),       # odd N
+    (100, 1000, 4096, 32, None, 4, 64),      # ragged last column block
+    (64, 1024, 8192, 64, None, 8, 64),
+    (200, 2600, 3072, 64, None, 2, 96),      # three blocks along M, ragged N
+    (400, 1300, 3072, 128, None, 2, 96),     # five, the last of 80 rows
+    (96, 5120, 3072, 64, None, 3, 96),       # Llama q|k|v at M = 96
+    (257, 777, 4096, 32, None, 4, 96),       # three blocks of 86, 86 and 85 rows
+    (257, 512, 10240, 64, None, 8, 96),
+    (200, 3072, 8192, 64, None, 2, 128),     # two blocks along M
+    (333, 1500, 6144, 64, None, 3, 128),
+    (128, 4096, 10240, 64, None, 4, 128),    # T5 wo at M = 128
+    # gated pairs
+    (70, 1001, 2048, 32, "silu", 2, 64),
+    (64, 1001, 3072, 64, "gelu", 3, 64),     # odd N
+    (96, 1024, 4096, 64, "silu", 4, 64),
+    (100, 333, 8192, 128, "gelu", 8, 64),
+    (333, 777, 3072, 64, "silu", 2, 96),
+    (96, 2560, 3072, 64, "gelu", 3, 96),
+    (333, 333, 4096, 32, "silu", 4, 96),
+    (96, 1000, 10240, 64, "gelu", 8, 96),
+    (128, 4096, 8192, 64, "silu", 2, 128),
+    (333, 777, 6144, 64, "gelu", 3, 128),
+    (400, 512, 8192, 64, "silu", 4, 128),
+    # unsplit (split three ways before M-blocks of 64 rows)
+    (128, 5120, 3072, 64, None, 1, 64),
+    (128, 2560, 3072, 64, "gelu", 1, 64),
 ]
-T5_WO, GELU_PAIR = CASES[4], CASES[9]
+T5_WO = (128, 4096, 10240, 64, None, 4, 128)
+PAIRS = [(64, 1001, 3072, 64, "gelu", 3, 64), (128, 4096, 8192, 64, "silu", 2, 128),
+         (96, 1000, 10240, 64, "gelu", 8, 96)]
 
 
 def _run(pkg, args, M, N, K, g, epi, out=None, stream=None, f32=False):
@@ -74,40 +76,41 @@ def _inputs(dev, M, N, K, g, epi, seed):
     return (x, sets), (to_dev(x, dev), [tuple(to_dev(a, dev) for a in w) for w in sets])
 
 
-@pytest.mark.parametrize("M,N,K,g,epi,splits", CASES)
-def test_wide_split_parity(pkg, dev, M, N, K, g, epi, splits):
+@pytest.mark.parametrize("M,N,K,g,epi,splits,rows", CASES)
+def test_wide_split_parity(pkg, dev, M, N, K, g, epi, splits, rows):
     import torch
-    assert wide_splits(M, N, K, g, epi is not None) == splits
-    assert pkg.gemm_route(M, N, K, group_size=g, gated=epi is not None) == "wide"
+    assert plan(pkg, M, N, K, g, epi is not None)[:3] == ("wide", splits, rows)
     (x, sets), args = _inputs(dev, M, N, K, g, epi, seed=M + N + K)
     y = _run(pkg, args, M, N, K, g, epi)
     again = [_run(pkg, args, M, N, K, g, epi) for _ in range(4)]
     torch.cuda.synchronize()
     for r in again:
         assert torch.equal(r, y)
-    rows = np.unique(np.array([0, 1, 31, 32, M // 2, M - 1]))
-    xs = x[rows].astype(np.float64)
+    at = np.unique(np.array([0, 1, 31, 32, M // 2, M - 1]))
+    xs = x[at].astype(np.float64)
     if epi is None:
         y32 = _run(pkg, args, M, N, K, g, epi, f32=True)
         torch.cuda.synchronize()
         assert torch.equal(y32.half(), y)
         want = o.matmul_q4_f64(xs, *sets[0], g)
-        assert_parity(y32.cpu().numpy()[rows], want, TOL_GEMM_F16, f"M={M} N={N} K={K} S={splits}")
+        assert_parity(y32.cpu().numpy()[at], want, TOL_GEMM_F16, f"M={M} N={N} K={K} S={splits}")
     else:
         gp = o.matmul_q4_f64(xs, *sets[0], g)
         up = o.matmul_q4_f64(xs, *sets[1], g)
         want = o.gelu_tanh_f64(gp) * up if epi == "gelu" else o.silu_mul_f64(gp, up)
-        got = y.cpu().numpy()[rows].astype(np.float64)
+        got = y.cpu().numpy()[at].astype(np.float64)
         assert o.max_rel_err(got, want) <= GATE, f"{epi} M={M} N={N} K={K} S={splits}"
 
 
 def test_wide_splits_back_to_back(pkg, dev):
-    """Split launches of three shapes with different tile counts and split
+    """Split launches of four shapes with different tile counts and split
     counts, interleaved on one stream with no synchronization between them
-    (120 launches): each launch must leave every counter at zero for the
+    (160 launches): each launch must leave every counter at zero for the
     next, and each must equal the first bit for bit."""
     import torch
-    shapes = [CASES[0], T5_WO, CASES[5]]   # 3, 4 and 8 splits
+    # 3, 4, 8 and 2 splits
+    shapes = [(96, 5120, 3072, 64, None), T5_WO, (64, 1024, 8192, 64, None), (333, 777, 3072, 64, "silu")]
+    assert [plan(pkg, *c[:4], gated=bool(c[4])).splits for c in shapes] == [3, 4, 8, 2]
     inputs = [_inputs(dev, *c[:5], seed=7 + i)[1] for i, c in enumerate(shapes)]
     st = torch.cuda.Stream()
     with torch.cuda.stream(st):
@@ -125,7 +128,9 @@ def test_wide_splits_in_graph(pkg, dev):
     the same stream between the replays: every replay equals the eager
     results bit for bit."""
     import torch
-    shapes = [T5_WO, GELU_PAIR]
+    shapes = [T5_WO, *PAIRS]
+    for M, N, K, g, epi, splits, rows in shapes:
+        assert plan(pkg, M, N, K, g, epi is not None)[:3] == ("wide", splits, rows)
     inputs = [_inputs(dev, *c[:5], seed=21 + i)[1] for i, c in enumerate(shapes)]
     st = torch.cuda.Stream()
     with torch.cuda.stream(st):

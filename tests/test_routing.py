@@ -9,6 +9,8 @@ import pytest
 import test_gpu_mid
 import test_gpu_narrow
 import test_gpu_skinny
+import test_gpu_wide_splits
+from helpers import plan
 
 LLAMA_PAIR = dict(N=8192, K=3072, gated=True)
 T5_WI_PAIR = dict(N=10240, K=4096, gated=True)
@@ -165,3 +167,23 @@ def test_small_m_parity_shapes_run_the_small_m_route(pkg):
 def test_mid_parity_shapes_run_the_mid_route(pkg):
     for M, N, K, g in test_gpu_mid.SHAPES:
         assert pkg.gemm_route(M, N, K, group_size=g) == "mid", (M, N, K, g)
+
+
+# The GPU tests whose shapes are there for a plan: a planner that moves them off
+# it shows here.
+
+def test_wide_split_cases(pkg):
+    """Each case runs the plan it names, and each (pair, splits, block height) the
+    planner takes over these shapes has a case."""
+    for M, N, K, g, epi, splits, rows in test_gpu_wide_splits.CASES:
+        assert plan(pkg, M, N, K, g, epi is not None)[:3] == ("wide", splits, rows), (M, N, K, g, epi)
+    planned = set()
+    for M in (33, 64, 65, 96, 97, 128, 200, 256, 257, 333, 400, 500):
+        for N in (33, 333, 512, 777, 1000, 1300, 1500, 2048, 2560, 3072, 4096, 5120):
+            for K in (1920, 2048, 2560, 3072, 4096, 5120, 6144, 8192, 10240):
+                for pair in (False, True):
+                    p = plan(pkg, M, N, K, 64, pair)
+                    if p.route == "wide" and p.splits > 1:
+                        planned.add((pair, p.splits, p.rows))
+    cases = {(c[4] is not None, c[5], c[6]) for c in test_gpu_wide_splits.CASES}
+    assert planned <= cases, planned - cases
