@@ -379,8 +379,8 @@ def test_matmul_residual_rms_norm(pkg, dev, M, N, K, g, sum_rounded):
 @pytest.mark.parametrize("K", [3072, 8192])
 @pytest.mark.parametrize("sum_rounded", [False, True])
 def test_matmul_residual_rms_norm_equals_unfused(pkg, dev, K, sum_rounded):
-    """At the prefill shapes (M = 750, N = 3072; split-K in both plans) the fused
-    call equals, bit for bit, this library's unfused sequence: the GEMM, then
+    """At the prefill shapes (M = 750, N = 3072; K = 8192 splits K, K = 3072 does
+    not; every split count: test_gpu_residual_norm_routes.py) the fused call equals, bit for bit, this library's unfused sequence: the GEMM, then
     sltx_residual_rms_norm (o_proj step) or the residual GEMM epilogue and
     sltx_rms_norm (down_proj step and the next input norm).  Also in place
     (residual_out == residual)."""

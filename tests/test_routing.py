@@ -8,6 +8,7 @@ import pytest
 
 import test_gpu_mid
 import test_gpu_narrow
+import test_gpu_residual_norm_routes
 import test_gpu_skinny
 import test_gpu_wide_splits
 from helpers import plan
@@ -187,3 +188,12 @@ def test_wide_split_cases(pkg):
                         planned.add((pair, p.splits, p.rows))
     cases = {(c[4] is not None, c[5], c[6]) for c in test_gpu_wide_splits.CASES}
     assert planned <= cases, planned - cases
+
+
+def test_split_residual_norm_cases(pkg):
+    """Also: the pass has a case for each of its row lengths and split counts."""
+    cases = test_gpu_residual_norm_routes.SPLIT
+    for M, N, K, g, splits in cases:
+        assert plan(pkg, M, N, K, g)[:2] == ("gemm", splits), (M, N, K, g)
+    passes = {(next(n for n in (2048, 4096, 8192, 16384) if c[1] <= n), min(c[4], 5)) for c in cases}
+    assert passes == {(n, s) for n in (2048, 4096, 8192, 16384) for s in (2, 3, 4, 5)}
