@@ -7,23 +7,29 @@ branch, DiTModel.swift:102-125) and, where its grid ends, against the GEMM."""
 import numpy as np
 import pytest
 
-from helpers import TOL_GEMM_F16, assert_parity, host
+from helpers import TOL_GEMM_F16, assert_parity, host, plan
 from oracle import q4_oracle as o
 
 pytestmark = pytest.mark.gpu
 
 
-# 32-row blocks up to 8192 / ceil(N / 128) rows, then 64-row ones up to twice
-# that, then the GEMM; K > 2048 from M N = 2^18
-SHAPES = [(1, 128, 128, 64), (31, 1, 256, 32), (33, 130, 2048, 32), (777, 127, 1152, 128),
-          (6144, 128, 2048, 64), (8192, 100, 128, 64), (8193, 100, 128, 64), (4097, 256, 2048, 32),
-          (2731, 384, 384, 128), (2700, 512, 640, 64), (16384, 65, 128, 128), (16385, 65, 128, 128),
-          (2048, 128, 4096, 64), (600, 500, 3072, 128), (500, 500, 4096, 64)]
+# (M, N, K, g, rows of a block; 0: past the kernel's limits, the GEMM).  32-row
+# blocks up to 8192 / ceil(N / 128) rows, then 64-row ones up to twice that; K %
+# 128 == 0 and at most 64 groups; K > 2048 from M N = 2^18.
+SHAPES = [(1, 128, 128, 64, 32), (31, 1, 256, 32, 32), (33, 130, 2048, 32, 32), (777, 127, 1152, 128, 32),
+          (6144, 128, 2048, 64, 32), (8192, 100, 128, 64, 32), (8193, 100, 128, 64, 64),
+          (4096, 256, 2048, 32, 32), (4097, 256, 2048, 32, 64), (2731, 384, 384, 128, 64),
+          (2700, 512, 640, 64, 64), (16384, 65, 128, 128, 64), (16385, 65, 128, 128, 0),
+          (4096, 512, 2048, 64, 64), (4097, 512, 2048, 64, 0), (2048, 128, 4096, 64, 32),
+          (2047, 128, 4096, 64, 0), (600, 500, 3072, 128, 32), (500, 500, 4096, 64, 0),
+          (600, 500, 4224, 128, 0), (600, 500, 2176, 32, 0), (100, 128, 2080, 32, 0)]
 
 
-@pytest.mark.parametrize("M,N,K,g", SHAPES)
-def test_strip(pkg, dev, M, N, K, g):
+@pytest.mark.parametrize("M,N,K,g,block", SHAPES)
+def test_strip(pkg, dev, M, N, K, g, block):
     import torch
+    got = plan(pkg, M, N, K, g, x_dtype=torch.float32)
+    assert got.route == "gemm" and (got.rows == block if block else got.rows >= 128)
     gen = torch.Generator(device=dev).manual_seed(M + N + K)
     x = torch.randn(M, K, generator=gen, device=dev)
     x[M // 2, K // 3] = 1e6          # clamped

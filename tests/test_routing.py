@@ -10,6 +10,7 @@ import test_gpu_mid
 import test_gpu_narrow
 import test_gpu_residual_norm_routes
 import test_gpu_skinny
+import test_gpu_strip
 import test_gpu_wide_splits
 from helpers import plan
 
@@ -197,3 +198,10 @@ def test_split_residual_norm_cases(pkg):
         assert plan(pkg, M, N, K, g)[:2] == ("gemm", splits), (M, N, K, g)
     passes = {(next(n for n in (2048, 4096, 8192, 16384) if c[1] <= n), min(c[4], 5)) for c in cases}
     assert passes == {(n, s) for n in (2048, 4096, 8192, 16384) for s in (2, 3, 4, 5)}
+
+
+def test_strip_cases(pkg):
+    import torch
+    for M, N, K, g, block in test_gpu_strip.SHAPES:
+        p = plan(pkg, M, N, K, g, x_dtype=torch.float32)
+        assert p.route == "gemm" and (p.rows == block if block else p.rows >= 128), (M, N, K, g, p)
