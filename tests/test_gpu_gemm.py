@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from helpers import (TOL_GEMM_BF16, TOL_GEMM_F16, TOL_ROUNDED_W, TOL_GEMV, assert_parity,
-                     gpu_inputs, host, load_golden, q4w, rounded_weights_bf16,
+                     gpu_inputs, host, load_golden, plan, q4w, rounded_weights_bf16,
                      rounded_weights_f16, to_dev)
 from oracle import q4_oracle as o
 
@@ -245,9 +245,12 @@ def test_dit_ffn_m6144_bf16(pkg, dev):
 # fp32 partials in split order, then applies the epilogue) ----
 
 @pytest.mark.parametrize("M,N,K,xdt,epi,out", [
-    (40, 300, 4096, "f16", 2, "f16"),      # 2 tiles x 8 splits, bias + GELU
+    (40, 300, 4096, "f16", 2, "f16"),      # (the wide-M route, split) bias + GELU
+    (300, 3000, 4352, "f16", 2, "f16"),    # 128 x 128 tiles, bias + GELU
+    (130, 5000, 4352, "f16", 0, "f32"),    # 128 x 256 tiles
+    (40, 300, 4160, "f16", 2, "f16"),      # the generic GEMM, bias + GELU
     (130, 200, 8192, "bf16", 0, "f32"),    # bf16 activations, fp32 out
-    (7, 96, 2048, "f16", 0, "f16"),
+    (7, 96, 2048, "f16", 0, "f16"),        # (the small-M route)
 ])
 def test_gemm_split_k(pkg, dev, M, N, K, xdt, epi, out):
     import torch
@@ -273,24 +276,40 @@ def test_gemm_split_k(pkg, dev, M, N, K, xdt, epi, out):
     assert np.all(np.abs(y - ref) <= allow), float(np.max(np.abs(y - ref) / allow))
 
 
-@pytest.mark.parametrize("M,N,K", [(64, 256, 4096), (3, 128, 8192)])
+# (the wide-M and the small-M route; the GEMM's 128- and 256-row weight tiles and
+# its generic kernel)
+@pytest.mark.parametrize("M,N,K", [(64, 256, 4096), (3, 128, 8192), (300, 1500, 4352), (257, 1500, 4352),
+                                   (64, 256, 4160)])
 def test_swiglu_gemm_split_k(pkg, dev, M, N, K):
     import torch
     g = 64
+    if K > 4096 and K < 8192:
+        p = plan(pkg, M, N, K, gated=True)
+        assert p.route == "gemm" and p.splits > 1
     x, [(wg, sg, bg), (wu, su, bu)] = o.make_inputs(M, N, K, g, seed=N + K, n_weights=2)
     ref = o.silu_mul_f64(o.matmul_q4_f64(x, wg, sg, bg, g), o.matmul_q4_f64(x, wu, su, bu, g))
     y = pkg.matmul_q4_silu_mul(to_dev(x, dev), q4w(pkg, wg, sg, bg, K, g, dev),
                                q4w(pkg, wu, su, bu, K, g, dev), M, K, N)
     torch.cuda.synchronize()
-    assert_parity(y.cpu().numpy(), ref, TOL_GEMM_F16, f"swiglu split M={M}")
+    tol = TOL_GEMM_F16
+    if N > 256:
+        # many outputs: the weights rounded as the kernel rounds them (their rounding
+        # compounds in gate x up), which leaves fp32 sums, exp2 / rcp and one fp16 rounding
+        xs = x.astype(np.float64)
+        ref = o.silu_mul_f64(xs @ rounded_weights_f16(wg, sg, bg, g).T, xs @ rounded_weights_f16(wu, su, bu, g).T)
+        tol = dict(rtol=1e-3, atol_rms=1e-4)
+    assert_parity(y.cpu().numpy(), ref, tol, f"swiglu split M={M}")
 
 
-def test_split_k_under_graph_capture(pkg, dev):
+@pytest.mark.parametrize("M,N,K,route,splits", [(16, 256, 4096, "small_m", 1), (300, 3000, 4352, "gemm", 3),
+                                                (257, 777, 4096, "wide", 4)])
+def test_split_k_under_graph_capture(pkg, dev, M, N, K, route, splits):
     """A split-K GEMM captured in a graph (workspace allocated by an eager call
     first) replays to the eager result; a fresh stream captured cold runs
-    unsplit and still matches."""
+    unsplit (a split wide-M launch: as the GEMM) and still matches."""
     import torch
-    M, N, K, g = 16, 256, 4096, 64
+    g = 64
+    assert plan(pkg, M, N, K, g)[:2] == (route, splits)
     x, [(w, s, b)] = o.make_inputs(M, N, K, g, seed=12)
     tx, qw = to_dev(x, dev), q4w(pkg, w, s, b, K, g, dev)
     ref = pkg.matmul_q4_fast_f32(tx, qw.weight, qw.scales, qw.biases, M, K, N, g)
@@ -316,11 +335,12 @@ def test_split_k_under_graph_capture(pkg, dev):
 
 
 @pytest.mark.parametrize("kind", ["plain", "silu", "residual", "f32_bias_gelu"])
-@pytest.mark.parametrize("M,N,K", [(33, 256, 512), (750, 3072, 8192)])
+@pytest.mark.parametrize("M,N,K", [(33, 256, 512), (257, 6000, 256), (750, 3072, 8192)])
 def test_unaligned_outputs_match_aligned(pkg, dev, kind, M, N, K):
     """Outputs (and the residual input) 2 bytes (fp16) or 4 bytes (fp32) off a
-    16-byte boundary take the per-element store path of the staged epilogue
-    (and of the split-K reduction at M=750, K=8192); the values must be
+    16-byte boundary take the per-element store path of the wide-M route
+    (M=33), the GEMM's staged epilogue (M=257; a pair: the register one) and the
+    split-K reduction (M=750, K=8192); the values must be
     bit-identical to the aligned run's."""
     import torch
     x, [(w, s, b), (w2, s2, b2)] = gpu_inputs(M, N, K, 64, seed=M + K, dev=dev, n_weights=2)
@@ -352,13 +372,16 @@ def test_unaligned_outputs_match_aligned(pkg, dev, kind, M, N, K):
     assert torch.equal(aligned, unaligned), kind
 
 
+@pytest.mark.parametrize("M,N,K", [(70, 320, 1024), (257, 3000, 256), (257, 6000, 256)])
 @pytest.mark.parametrize("kind", ["f16", "silu", "bf16"])
-def test_scales_biases_at_2_byte_offset(pkg, dev, kind):
+def test_scales_biases_at_2_byte_offset(pkg, dev, kind, M, N, K):
     """Scales and biases 2 bytes off a 4-byte boundary (allowed: 2-byte
-    alignment) cannot move as dword pairs, so the launcher routes them to the
-    generic kernel; the values must match the aligned run and the oracle."""
+    alignment) cannot move as dword pairs, so the GEMM (bf16; at M = 257 the pair
+    of 3000 and the single set of 6000 columns too) takes its generic kernel for
+    them, and the wide-M route reads them as 16-bit values anyway; the values
+    must match the aligned run and the oracle."""
     import torch
-    M, N, K, g = 70, 320, 1024, 64
+    g = 64
     x, sets = gpu_inputs(M, N, K, g, seed=17, dev=dev, n_weights=2,
                          x_dtype="bf16" if kind == "bf16" else "f16")
 
@@ -392,6 +415,15 @@ def test_scales_biases_at_2_byte_offset(pkg, dev, kind):
     else:
         ref = o.matmul_q4_f64(xh, *hs[0], g)
         tol = TOL_GEMM_F16
+    if M > 70:
+        # many outputs: the weights rounded as the kernel rounds them, which leaves the
+        # fp32 sums and the epilogue (a pair: exp2 / rcp) and output rounding
+        if kind == "bf16":
+            ref = o.bf16_bits_to_f32(xh).astype(np.float64) @ rounded_weights_bf16(*hs[0], g).T
+        else:
+            ys = [xh.astype(np.float64) @ rounded_weights_f16(*t, g).T for t in hs]
+            ref = o.silu_mul_f64(*ys) if kind == "silu" else ys[0]
+        tol = dict(rtol=1e-3, atol_rms=1e-4) if kind == "silu" else TOL_ROUNDED_W
     assert_parity(yu.float().cpu().numpy(), ref, tol, f"2-byte-offset scales {kind}")
     assert_parity(ya.float().cpu().numpy(), ref, tol, f"aligned scales {kind}")
     ok, worst = o.elementwise_ok(yu.float().cpu().numpy(), ya.float().cpu().numpy().astype(np.float64),

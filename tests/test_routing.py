@@ -6,6 +6,7 @@ small-M kernel rely on.
 """
 import pytest
 
+import test_gpu_gemm_groups
 import test_gpu_mid
 import test_gpu_narrow
 import test_gpu_residual_norm_routes
@@ -205,3 +206,10 @@ def test_strip_cases(pkg):
     for M, N, K, g, block in test_gpu_strip.SHAPES:
         p = plan(pkg, M, N, K, g, x_dtype=torch.float32)
         assert p.route == "gemm" and (p.rows == block if block else p.rows >= 128), (M, N, K, g, p)
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+def test_gemm_tile_cases(pkg, g):
+    for pair, cases in ((False, test_gpu_gemm_groups.TILES), (True, test_gpu_gemm_groups.PAIR_TILES)):
+        for c in cases:
+            assert test_gpu_gemm_groups._runs_tile(pkg, *c[:3], g, pair, *c[3:]), (c, g)
