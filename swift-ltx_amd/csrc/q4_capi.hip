@@ -976,7 +976,8 @@ int sltx_gemm_route(int32_t M, int32_t N, int32_t K, int32_t group_size, int32_t
 // For the tests, and so not in the public header: what run_gemm plans, as
 // {sltx_gemm_route, K splits across blocks, and, of the wide route, the GEMM and
 // its strip kernel (the one with fewer than 128 rows), the activation and the
-// weight rows of a block, else 0}.
+// weight rows of a block; of the small-M route, where X comes from (SkinnyX) and
+// the weight rows; else 0}.
 int sltx_internal_plan(int32_t M, int32_t N, int32_t K, int32_t group_size, int32_t gated, int32_t x_dtype,
                        int32_t out[4]) {
     GemmParams p;
@@ -988,7 +989,10 @@ int sltx_internal_plan(int32_t M, int32_t N, int32_t K, int32_t group_size, int3
     out[0] = gemm_route(p, x_dtype == kBF16, &np, &sp, &wp);
     out[1] = 1;
     out[2] = out[3] = 0;
-    if (out[0] == SLTX_ROUTE_MID) {
+    if (out[0] == SLTX_ROUTE_SMALL_M) {
+        out[2] = sp.XM;
+        out[3] = 16 * sp.RT;
+    } else if (out[0] == SLTX_ROUTE_MID) {
         out[1] = mid_splits(p);
     } else if (out[0] == SLTX_ROUTE_WIDE) {
         out[1] = wp.splits;

@@ -23,15 +23,14 @@
 //    memory path costs that path 16 cycles whatever its lanes hold, so
 //    fragments loaded for all 16 rows (zeros past M) cost the CU more load
 //    issue than its weights at small M.  Hence three ways (SkinnyX):
-//    - M <= 8 (kXHalf): the lanes of rows 8..15 load rows 0..7 of the next
+//    - M <= 8 (kXHalf), but for the shapes of skinny_plan's rule: the lanes of rows 8..15 load rows 0..7 of the next
 //      fragment, so that one load fills two; a row rotation by 8 lanes (DPP)
 //      gives the second.  The tile's rows 8..15 then hold other rows' data,
 //      which reaches only outputs that are not stored.  Against X in LDS at
 //      M = 8: Llama down 10.2 -> 9.5 us, 16384 x 4096 16.9 -> 13.2, 12000 x
-//      6144 21.7 -> 17.7, the gate/up pairs and q|k|v within 2%; and half the
-//      X registers, so that 16 waves reach K = 14336 (4096 rows at M = 2 / 8:
+//      6144 21.7 -> 17.7; and half the X registers, so that 16 waves reach K = 14336 (4096 rows at M = 2 / 8:
 //      13.0 / 16.9 us against the GEMM's 32).
-//    - one tile of 9..16 rows that fit (kXLds): the block first copies the M
+//    - one tile of 9..16 rows that fit, and those shapes (kXLds): the block first copies the M
 //      real rows to LDS (rows padded by 16 bytes: the 16 rows of a fragment
 //      read hit distinct banks), before its weight loads, and each wave reads
 //      its fragments from there; rows past M read row 0.
@@ -419,10 +418,20 @@ bool skinny_plan(const GemmParams& p, bool a_bf16, SkinnyPlan* out) {
     // X of 9..16 rows in LDS: where the rows fit beside the slabs, so that a
     // block still gets its share of the CU's LDS (all of it where the grid has
     // no second block for a CU: 3072 x 3072 at M = 16 takes 5.6 us with X in
-    // LDS, 6.2 without).
-    if (pl.W == 8 && mt == 1 && pl.XM == kXRegs &&
-        skinny_lds(p, pl.RT, pair, true) <=
-            (size_t)(pl.RT == 2 || (p.N + 15) / 16 <= kCUs ? 128 : 64) * 1024)
+    // LDS, 6.2 without).  Of at most 8 rows too, where blocks of three steps, or
+    // of two of one set, share CUs (at one step and from four, at one block per CU
+    // and for pairs of group 32, whose scales fill more of the LDS, halves are the
+    // faster).  Measured, LDS against halves: 5120 x 3072 at M
+    // = 5 / 6 / 8 6.27 / 6.32 / 6.77 us against 6.51 / 6.80 / 7.34, the gate/up pair at
+    // M = 2 / 4 / 6 / 8 9.05 / 9.40 / 9.56 / 9.85 against 9.09 / 9.70 / 9.88 / 10.28, 5120 x
+    // 2048 at M = 5 / 8 4.72 / 4.96 against 5.01 / 5.52; pairs of two steps at M = 5 / 8
+    // 6.96 / 7.19 against 6.67 / 7.17, the gate/up pair of group 32 at M = 2 / 8 9.80 /
+    // 10.57 against 9.28 / 10.72, 8000 x 1024 at M = 5 3.85 / 3.74, 8000 x 4096 8.18 / 8.02.
+    const long blocks = (p.N + 16L * pl.RT - 1) / (16 * pl.RT);
+    const bool few_in_lds = blocks > kCUs && pl.RT == 1 &&
+                            (pair ? pl.STEPS == 3 && p.gshift > 0 : pl.STEPS == 3 || pl.STEPS == 2);
+    if (pl.W == 8 && mt == 1 && (pl.XM == kXRegs || few_in_lds) &&
+        skinny_lds(p, pl.RT, pair, true) <= (size_t)(pl.RT == 2 || blocks <= kCUs ? 128 : 64) * 1024)
         pl.XM = kXLds;
     // scales and biases are staged with 16-byte loads
     const uintptr_t sb = reinterpret_cast<uintptr_t>(p.s0) | reinterpret_cast<uintptr_t>(p.b0) |

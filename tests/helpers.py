@@ -105,7 +105,9 @@ def host(t):
 class Plan(NamedTuple):
     """The kernel family, its K splits across blocks, and (wide route, GEMM and
     strip kernel) the activation and weight rows of a block.  The strip kernel's
-    family is "gemm"; its 32 or 64 rows tell it from the GEMM's 128 or 192."""
+    family is "gemm"; its 32 or 64 rows tell it from the GEMM's 128 or 192.  The
+    small-M route gives for rows where X comes from (SkinnyX of q4_launch.hpp: 0
+    registers, 1 LDS, 2 halves)."""
     route: str
     splits: int
     rows: int

@@ -172,6 +172,25 @@ def test_mid_parity_shapes_run_the_mid_route(pkg):
         assert pkg.gemm_route(M, N, K, group_size=g) == "mid", (M, N, K, g)
 
 
+@pytest.mark.parametrize("M", [5, 6, 7, 8])
+def test_small_m_takes_x_from_lds_where_it_is_faster(pkg, M):
+    """At most 8 rows: halves, but LDS where blocks of three steps, or of two of one
+    set, share CUs (us in LDS / halves at M = 8: 5120 x 3072 6.77 / 7.34, the
+    gate/up pair 9.85 / 10.28; the pair at K = 2048, M = 5: 6.96 / 6.67, of group 32
+    at K = 3072, M = 2: 9.80 / 9.28)."""
+    x = lambda N, K, **kw: plan(pkg, M, N, K, **kw)[0::2]
+    lds, half = ("small_m", 1), ("small_m", 2)
+    for N in (4112, 5120, 8160):
+        assert x(N, 3072) == lds and x(N, 2048) == lds, N
+        assert x(N, 1024) == half and x(N, 4096) == half and x(N, 6144) == half, N
+        assert x(N, 3072, gated=True) == lds, N
+        for K in (1024, 2048, 4096):
+            assert x(N, K, gated=True) == half, (N, K)
+    assert x(8192, 3072, gated=True) == lds and x(8192, 3072, g=32, gated=True) == half
+    assert x(3072, 3072) == half and x(4096, 2048) == half      # one block per CU
+    assert x(32064, 3072) == half                               # two row tiles
+
+
 # The GPU tests whose shapes are there for a plan: a planner that moves them off
 # it shows here.
 
