@@ -902,10 +902,12 @@ int sltx_matmul_q4_residual_rms_norm(const void* x, const sltx_q4_weight* w, con
     // 13.7 / 15.8 / 19.5 / 24.8 / 33.0 against 23.2 / 23.6 / 24.7 / 26.2 / 29.8 /
     // 33.7.  An unsplit GEMM and the norm against split partials and the fused pass:
     // 2048 x 2048 at M = 500 / 1200 15.9 / 26.1 against 24.1 / 29.4, 4096 x 3072 at
-    // M = 700 / 1100 34.0 / 47.5 against 35.9 / 49.3; the slower one only around
-    // 4096 x 4096 at M = 700..1024 (44.8 - 53.3 against 43.8 - 52.4), where the
-    // unfused product is the faster unsplit (47 against 50) and both calls plan
-    // alike so that their results agree bit for bit.
+    // M = 700 / 1100 34.0 / 47.5 against 35.9 / 49.3; the slower one only at 4096 x
+    // 4096, M = 690..850, and there the unrounded form (43.2 / 44.0 / 47.4 against
+    // 42.0 / 42.8 / 47.0 at M = 700 / 768 / 850; rounded 42.1 / 43.3 / 46.5 against 42.0 /
+    // 42.8 / 46.9): the product alone is the faster unsplit (37.8 / 38.7 / 42.3 against
+    // 40.2 / 41.0 / 44.2), and both calls plan alike so that their results agree bit
+    // for bit.
     // (Under capture without a workspace the call has already failed,
     // as it does for every shape.)
     NarrowPlan np;

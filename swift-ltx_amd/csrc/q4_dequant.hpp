@@ -1,5 +1,5 @@
 // q4_dequant.hpp -- the register dequantization shared by the MFMA kernels
-// (q4_gemm.hip, q4_mid.hip, q4_skinny.hip, q4_narrow.hip): one packed word of
+// (q4_gemm_kernel.hpp, q4_mid.hip, q4_skinny.hip, q4_narrow.hip): one packed word of
 // 8 nibbles -> 8 fp16 weights s * q + b, each rounded once (matmulQ4Fast's
 // fp16 dequant, Ops.swift:312-381), in k order or in an order that a matching
 // reorder of 8 activations follows, and the XOR-swizzled 128-byte LDS rows

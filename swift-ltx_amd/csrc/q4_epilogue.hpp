@@ -1,5 +1,5 @@
 // q4_epilogue.hpp -- the MFMA kernels' output stage on eight consecutive
-// columns of one row (q4_gemm.hip, q4_wide.hip): the fp32 bias, GELU-tanh
+// columns of one row (q4_gemm_kernel.hpp, q4_wide.hip): the fp32 bias, GELU-tanh
 // and residual epilogues, 16-byte vector stores when the row allows them, and
 // raw fp32 partial sums for split-K workspaces.
 #pragma once

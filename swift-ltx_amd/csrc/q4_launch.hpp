@@ -44,7 +44,7 @@ bool gemv2_ok(int N, int K);
 
 enum GemvPro : int { kProNone = 0, kProRms = 1, kProResidualRms = 2 };
 
-// GEMM (M > 1) operands; see q4_gemm.hip.
+// GEMM (M > 1) operands; see q4_gemm_kernel.hpp.
 struct GemmParams {
     const void* a;          // [M, K] fp16 or bf16
     const uint32_t* w0;     // [N, K/8]
@@ -68,7 +68,8 @@ struct GemmParams {
     unsigned* tickets;
     int splits;             // filled by launch_gemm
     int split_tiles;        // k-tiles per split (even), filled by launch_gemm
-    uint32_t nib_mask;      // 0x0F0F0F0F, set by the launchers (a run-time value: see q4_gemm.hip)
+    uint32_t nib_mask;      // 0x0F0F0F0F, set by the launchers (a run-time value: see
+                            // dequant_word_bf16)
     int a_f32;              // a is fp32, cast to fp16 with the +-65504 clamp as it is staged (GEMM only)
 };
 

@@ -2,7 +2,7 @@
 // (T5 encoder layers at short sequence lengths, short prompts, batched
 // decode) on CDNA4 MFMA, as a weight stream.
 //
-// Same product as q4_gemm.hip, Y[M,N] = X[M,K] . dequant(W)[N,K]^T with fp32
+// Same product as q4_gemm_kernel.hpp, Y[M,N] = X[M,K] . dequant(W)[N,K]^T with fp32
 // accumulation (matmulQ4Fast, Ops.swift:312-381).  At these M a weight byte
 // feeds at most 32 multiply-adds, so the kernel should run at the weight
 // stream's rate; what it must not do is load X badly.  X is M x K fp16 (up to
@@ -35,7 +35,7 @@
 //    its own copies: s_waitcnt counts a wave's memory operations in issue
 //    order, so a wave that issued both streams would wait for weights issued
 //    before the X copy it needs.
-//  * Inside a k-tile the k order is permuted as in q4_gemm.hip: k-step s of
+//  * Inside a k-tile the k order is permuted as in q4_gemm_kernel.hpp: k-step s of
 //    lane half h is packed word 4h + s of the row, so a lane's B fragments
 //    over the k-tile are one 16-byte piece, dequantized in registers
 //    (v_perm_b32 byte pairing, v_cvt_scalef32_pk_f16_fp8, one v_pk_fma_f16

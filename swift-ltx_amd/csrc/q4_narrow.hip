@@ -3,7 +3,7 @@
 // tokens) on CDNA4's 4x4x4 MFMA blocks, as a weight stream shaped like the
 // GEMV.
 //
-// Same product as q4_gemm.hip, Y[M,N] = X[M,K] . dequant(W)[N,K]^T with the
+// Same product as q4_gemm_kernel.hpp, Y[M,N] = X[M,K] . dequant(W)[N,K]^T with the
 // weights dequantized to fp16 (s * q + b, one rounding) and fp32 accumulation
 // (matmulQ4Fast, Ops.swift:312-381).  At M <= 4 each weight byte feeds at
 // most 4 multiply-adds: the launch is bound by the weight stream, and what

@@ -1529,7 +1529,9 @@ size_t argmax_workspace_bytes() { return 2 * kMaxBlocks * 4; }
 // probabilities, block maxima and exp-sums, the level-0 and range
 // histograms (count, mass, key min and max), the control block, the tied-key
 // chunk counts, candidates
-constexpr size_t kHistBytes = 20 * kLevelBins;   // more than a histogram takes (20 kBins)
+// A histogram takes 20 kBins bytes; the space for one keeps its size at 4096 bins
+// (120 KB in all beside n * 12 bytes), and with it the scratch size stated below.
+constexpr size_t kHistBytes = 20 * kLevelBins;
 constexpr size_t sample_ws_bytes(size_t n) {
     return (n * 4 + 255) / 256 * 256 + 2 * ((kMaxBlocks * 4 + 255) / 256 * 256) +
            2 * kHistBytes + 256 +

@@ -2,7 +2,7 @@
 // short prompts, the T5 encoder's S <= 128 layers, batched decode) on CDNA4
 // MFMA, as a weight stream.
 //
-// Same product as q4_gemm.hip, Y[M,N] = X[M,K] . dequant(W)[N,K]^T with fp32
+// Same product as q4_gemm_kernel.hpp, Y[M,N] = X[M,K] . dequant(W)[N,K]^T with fp32
 // accumulation (matmulQ4Fast, Ops.swift:312-381).  At small M each weight
 // byte feeds only M multiply-adds, so the kernel is bound by the weight
 // stream, like the GEMV: the block tile of the large-M GEMM (128 or 192

@@ -3,7 +3,7 @@
 // T5Encoder.swift:72-78 and :140-205; prompts of up to some hundred tokens;
 // narrow projections of more) on CDNA4 MFMA.
 //
-// Same product as q4_gemm.hip, Y[M,N] = X[M,K] . dequant(W)[N,K]^T with fp32
+// Same product as q4_gemm_kernel.hpp, Y[M,N] = X[M,K] . dequant(W)[N,K]^T with fp32
 // accumulation (matmulQ4Fast, Ops.swift:312-381).  Between the mid-M weight
 // stream (M <= 32) and the large-M GEMM (128- or 192-row tiles of 256 weight
 // rows), the GEMM's tiles are too few to fill 256 CUs and its split-K fp32
@@ -513,9 +513,13 @@ hipError_t launch_tm(const GemmParams& p, const WideArgs& wa, const dim3& grid, 
 // 64 (that pair at M = 64: 34.8 against 37.3).
 //
 // The estimate, in us, from launches at K = 128..10240, M = 33..6144 and
-// 10..256 blocks (it is within 1 us of them): a fixed part (launch, first
-// memory latency, scale slab, cross-wave sum), a round of 128 k, dearer with
-// more rows and with more CUs pulling X from L2, and the splits' hand-off.
+// 10..256 blocks: a fixed part (launch, first memory latency, scale slab,
+// cross-wave sum), a round of 128 k, dearer with more rows and with more CUs
+// pulling X from L2, and the splits' hand-off.  Over 187 one-round shapes
+// replayed in a graph it is 1.3 us high at the median (a launch costs less
+// there), from 2.5 low (the gate/up pair at M = 96, 256 blocks: 19.0 for 21.4)
+// to 3.6 high (2048 x 8192 at M = 33, 8 splits: 16.1 for 12.5); two rounds are
+// 5 high (the T5 pair at M = 64: 39.8 for 35.2).
 // Against the tallest M-blocks that fit, as the plan was: o (3072 x 3072) at
 // M = 128 / 256 13.1 / 15.5 us (2 x 64 rows x 2 splits, 4 x 64 x 1) against
 // 15.6 / 17.4; 4096 x 4096 15.0 / 19.4 against 17.0 / 20.4; Llama down keeps

@@ -1,4 +1,4 @@
-"""GPU parity of the GEMM's persistent launches (q4_gemm.hip, PERSIST): more
+"""GPU parity of the GEMM's persistent launches (q4_gemm_kernel.hpp, PERSIST): more
 output tiles than one block per CU, on the fast path (group size 64,
 K % 256 == 0).  One block per CU walks a fixed list of tiles, the copy ring
 runs on across tile boundaries (the last three k-tiles of a tile copy the

@@ -5,9 +5,10 @@ against the same pipeline run in numpy from the oracle's functions
 rows, so every row depends on its own token only):
 
 * the last token's logits within the parity gate (max|d|/max|ref| <= 1e-2)
-  of the numpy pipeline, at prompt lengths that take the MFMA GEMM (M > 1,
-  split-K included) and the GEMV (M = 1, for q|k|v and gate/up; the fused o
-  and down calls run the GEMM at every M);
+  of the numpy pipeline, at prompt lengths that take the M > 1 routes (this
+  model's small K runs the GEMM and the wide-M route) and the GEMV (M = 1, for
+  q|k|v and gate/up; the fused o and down calls run the M > 1 product at M = 1
+  too);
 * row independence: the last row's logits do not depend on the other tokens;
 * a captured prefill replays with new token ids exactly as an eager run.
 """

@@ -1,6 +1,6 @@
-"""GPU parity of the wide-M route (q4_wide.hip: 32 < M <= 256, fp16
-activations) through the C ABI: single weight sets and gated pairs, one
-block along M (33..128 rows, 2-4 MFMA row tiles) and two (129..256 rows),
+"""GPU parity of the wide-M route (q4_wide.hip: 32 < M, fp16 activations; here
+up to 256 rows, test_gpu_wide_rows.py beyond) through the C ABI: single weight
+sets and gated pairs, one block along M and several, of 2-4 MFMA row tiles each,
 unsplit and split over K across blocks (the last block of each output tile
 adds the splits' fp32 partial sums; tests/test_gpu_wide_splits.py covers
 that hand-over), every group size, the single-set epilogues.
